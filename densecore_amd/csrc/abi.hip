@@ -271,7 +271,7 @@ dc_status bwd_f32_chunked(const dc::BwdArgs &a, size_t avail, hipStream_t st) {
 size_t decode_ws(const dc::AttnShape &s, bool bf16) {
     if (s.E > dc::kDecodeMaxHeadDim) return dc::wide_ws_bytes(s, bf16, false);
     int split_len = 0;
-    const int splits = dc::decode_splits(s, &split_len);
+    const int splits = dc::decode_splits(s, bf16, &split_len);
     return round_up((size_t)s.B * s.H * splits * (s.E + 2) * sizeof(float));
 }
 
@@ -567,7 +567,7 @@ dc_status dc_sdpa_decode(const dc_attn_desc *d, const void *q, const void *k, co
     a.s = s;
     a.q = q, a.k = k, a.v = v, a.out = out, a.lse = lse;
     a.part = static_cast<float *>(workspace);
-    a.splits = dc::decode_splits(s, &a.split_len);
+    a.splits = dc::decode_splits(s, d->dtype == DC_BF16, &a.split_len);
     return decode_then_ref_rows(a, d->dtype == DC_BF16, static_cast<hipStream_t>(stream));
 }
 
@@ -601,7 +601,7 @@ dc_status dc_sdpa_decode_noalloc(const dc_attn_desc *d, const void *q, const voi
     a.q = q, a.k = k, a.v = v, a.out = out, a.lse = lse;
     st = launched(dc::decode_scratch(&a.part));  // the device address, never the array's name
     if (st != DC_OK) return st;
-    a.splits = dc::decode_splits(s, &a.split_len);
+    a.splits = dc::decode_splits(s, d->dtype == DC_BF16, &a.split_len);
     return decode_then_ref_rows(a, d->dtype == DC_BF16, static_cast<hipStream_t>(stream));
 }
 

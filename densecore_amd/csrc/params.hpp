@@ -176,7 +176,7 @@ hipError_t launch_bwd_bf16(const BwdArgs &a, hipStream_t st);
 // split this shape).
 size_t bwd_bf16_split_bytes(const AttnShape &s);
 hipError_t launch_decode(const DecodeArgs &a, bool bf16, hipStream_t st);
-int decode_splits(const AttnShape &s, int *split_len);
+int decode_splits(const AttnShape &s, bool bf16, int *split_len);
 // The allocation-free decode's scratch (a static device array in decode.hip): its size, and its
 // address on the current device (looked up with hipGetSymbolAddress once per device).
 constexpr size_t kDecodeScratchBytes = (size_t)16 << 20;
