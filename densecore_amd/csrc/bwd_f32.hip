@@ -1,9 +1,13 @@
-// Float32 attention backward on CDNA4 MFMA (v_mfma_f32_32x32x2_f32).
+// Float32 attention backward on CDNA4 MFMA: head dims up to 64 on the bf16 matrix cores (split
+// products, x3.hpp; key_tile_x3 below), 65 to 128 on v_mfma_f32_32x32x2_f32 / 16x16x4_f32.
+// Causal B8 H12 L1024 D64, forward and backward, float32 MFMAs -> split products: 468 -> 375 us; key
+// padding B16 H16 L512 D64 620 -> 395; full B8 H16 L1024 D64 983 -> 738.
 //
 // Computes what DenseCore's torch_attention::backward computes (src/torch_attention.rs:286-468):
 //   dsum = rowsum(dO * O);  P = exp(scale * q k^T + mask - lse) (0 where causal-masked);
 //   dV += P^T dO;  dP = dO V^T;  dS = P * (dP - dsum);  dQ += scale dS K;  dK += scale dS^T Q,
-// accumulating over the query heads that share a kv head (:321-324).  The blocking is its own:
+// accumulating over the query heads that share a kv head (:321-324).  The blocking is its own (the
+// float32 MFMA's tile; key_tile_x3 says what it does otherwise):
 //
 //   * a workgroup owns 128 keys of one (batch, kv head); each of its 4 waves owns 32 keys and
 //     keeps them in VGPRs (K and V as MFMA B operands) together with its dK^T and dV^T
@@ -31,10 +35,12 @@
 // shares: stored in per-range slots and added in range order by the reduction (or, with the
 // minimum workspace, added atomically).
 #include <algorithm>
+#include <type_traits>
 
 #include "bwd_common.hpp"
 #include "common.hpp"
 #include "params.hpp"
+#include "x3.hpp"
 
 namespace dc {
 namespace {
@@ -57,21 +63,14 @@ struct alignas(16) BwdSmem {
     float dsum[kBM];
 };
 
-// Threads of a backward workgroup: 8 waves of 16 keys at D = 128 (key_tile16), 4 waves of 32 keys
-// otherwise (key_tile).
-// At D = 128 a caller may ask for the forward's score order instead (AttnShape::consistent): the
-// 4-wave tile, one wave per SIMD.
-constexpr bool kSixteenKeys(int D) { return D == 128; }
+// Head dim 128 (65 to 128, zero-padded) has two float32 tiles: 8 waves of 16 keys (key_tile16), and 4
+// waves of 32 keys (key_tile) where a caller asks for the forward's score order
+// (AttnShape::consistent).  Waves per SIMD: two and one (one workgroup per CU either way).
 constexpr int layout_threads(bool k16) { return k16 ? 2 * kThreads : kThreads; }
-constexpr int bwd_threads(int D) { return layout_threads(kSixteenKeys(D)); }
-// Waves per SIMD the kernels are built for: the 8-wave tile two (one workgroup per CU); the 4-wave
-// tile at D = 128 one; below, two without a mask (two 4-wave workgroups), one with.
-constexpr int bwd_waves_per_eu(int D, bool mask, bool k16) {
-    return k16 ? 2 : (D == 128 ? 1 : (mask ? 1 : 2));
-}
+constexpr int bwd_waves_per_eu(bool k16) { return k16 ? 2 : 1; }
 
 // Register staging of one step's Q and dO rows (fast path: E == D, 16-byte aligned).
-template <int D, int NT = bwd_threads(D)>
+template <int D, int NT>
 struct QStage {
     static constexpr int C4 = D / 4;
     static constexpr int N = kBM * C4 / NT;
@@ -284,36 +283,27 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
     const float *kb = static_cast<const float *>(a.k) + (int64_t)bhk * s.S * s.E;
     const float *vb = static_cast<const float *>(a.v) + (int64_t)bhk * s.S * s.E;
 
-    // K and V rows of this lane's key: K[key][g*DH + t], V[key][g*DH + t].
-    // At D = 128 the K row is not held in registers: S reads it from the workgroup's transposed
-    // K tile in LDS (which the dQ product needs anyway), one ds_read_b32 of 32 consecutive keys
-    // per half-wave and MFMA.  K and V rows plus the dK / dV accumulators (4 x 64 floats per lane)
-    // would not fit one wave's registers without spills.
-    constexpr bool KREG = D <= 64;
-    float kreg[KREG ? DH : 1], vreg[DH];
+    // V row of this lane's key: V[key][g*DH + t].  The K row is not held in registers: S reads it from
+    // the workgroup's transposed K tile in LDS (which the dQ product needs anyway), one ds_read_b32
+    // of 32 consecutive keys per half-wave and MFMA.  K and V rows plus the dK / dV accumulators
+    // (4 x 64 floats per lane) would not fit one wave's registers without spills.
+    float vreg[DH];
     const int ptid = opaque_index(tid);  // the prologue's own copy (see opaque_index)
     const int pkey = kw0 + (ptid & 31), pg = (ptid & 63) >> 5;
     {
-        const float *kr = kb + (int64_t)pkey * s.E, *vr = vb + (int64_t)pkey * s.E;
+        const float *vr = vb + (int64_t)pkey * s.E;
         if (VEC && pkey < s.S) {
 #pragma unroll
             for (int t = 0; t < DH; t += 4) {
                 const f32x4 y = *reinterpret_cast<const f32x4 *>(vr + pg * DH + t);
 #pragma unroll
                 for (int u = 0; u < 4; ++u) vreg[t + u] = y[u];
-                if constexpr (KREG) {
-                    const f32x4 x = *reinterpret_cast<const f32x4 *>(kr + pg * DH + t);
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) kreg[t + u] = x[u];
-                }
             }
         } else {
 #pragma unroll
             for (int t = 0; t < DH; ++t) {
                 const int d = pg * DH + t;
-                const bool ok = pkey < s.S && d < s.E;
-                if constexpr (KREG) kreg[t] = ok ? kr[d] : 0.f;
-                vreg[t] = ok ? vr[d] : 0.f;
+                vreg[t] = pkey < s.S && d < s.E ? vr[d] : 0.f;
             }
         }
     }
@@ -403,7 +393,7 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
             const f32x4 oo = *reinterpret_cast<const f32x4 *>(&sm.dout[lr][g * DH + t4]);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const float kk = KREG ? kreg[KREG ? t4 + u : 0] : sm.kt[g * DH + t4 + u][wave * 32 + lr];
+                const float kk = sm.kt[g * DH + t4 + u][wave * 32 + lr];
                 sacc = mfma_f32(qq[u], kk, sacc);
                 pacc = mfma_f32(oo[u], vreg[t4 + u], pacc);
             }
@@ -511,6 +501,503 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
     }
 }
 
+// The steps [i0, i1) of a key tile in plain float32 arithmetic, for key_tile_x3's tiles whose sums
+// were not finite: the wave's accumulator (dV of its keys for the first four waves, dK for the
+// others, in MFMA layout) and the tile's dQ slot rows (with float atomics the shares are in dq
+// already and stay).  Slow and rare.
+template <int D, bool CAUSAL, int MASK>
+DEVI void redo_key_tile(const BwdArgs &a, int tid, int bhk, int kt, int i0, int i1, f32x16 (&acc)[D / 32]) {
+    const AttnShape &s = a.s;
+    const int wave = tid >> 6, lane = tid & 63, lr = lane & 31, g = lane >> 5;
+    const int b = bhk / s.Hkv, hk = bhk % s.Hkv, n0 = kt * kBN;
+    const float *kb = static_cast<const float *>(a.k) + (int64_t)bhk * s.S * s.E;
+    const float *vb = static_cast<const float *>(a.v) + (int64_t)bhk * s.S * s.E;
+    const int m_begin = tile_m_begin(CAUSAL, kt), per_head = tile_per_head(s, kt);
+    const int rf = slot_from(s, kt);
+    const int64_t slot0 = slot_before(s, kt) * ((int64_t)s.B * s.H);
+    // P and dS of (query row, key), every lane its own pair.
+    auto pair = [&](int bh, int qq, int key, float &p, float &ds) {
+        const int64_t row = (int64_t)bh * s.L + qq;
+        const float *q = static_cast<const float *>(a.q) + row * s.E, *go = static_cast<const float *>(a.dout) + row * s.E;
+        const int kk = min(key, s.S - 1);
+        const float *kr = kb + (int64_t)kk * s.E, *vr = vb + (int64_t)kk * s.E;
+        float x = 0.f, dp = 0.f;
+#pragma unroll 4
+        for (int d = 0; d < s.E; ++d) x = fmaf(q[d], kr[d], x), dp = fmaf(go[d], vr[d], dp);
+        x *= s.scale;
+        if (MASK) x += s.mask[(int64_t)b * s.msb + (int64_t)(bh - b * s.H) * s.msh + (int64_t)qq * s.msl + kk];
+        p = exp2_fast((x - a.lse[row]) * kLog2e);
+        if (key >= s.S || (CAUSAL && key > qq)) p = 0.f;
+        ds = p * (dp - a.dsum[row]);
+    };
+    const bool values = wave < 4;  // this wave's accumulator: dV, or dK
+    const int kw0 = n0 + (wave & 3) * 32;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+    for (int i = i0; i < i1; ++i) {
+        const int bh = b * s.H + hk * s.repeat + i / per_head, m0 = m_begin + (i % per_head) * kBM;
+        for (int qq = m0; qq < min(m0 + kBM, s.L); ++qq) {
+            const int64_t row = (int64_t)bh * s.L + qq;
+            // dQ: the waves take the rows in turn, lanes the tile's keys, then lanes the dims.
+            if (a.dq_part && (qq & 7) == wave) {
+                float p, d0, d1, t = 0.f;
+                pair(bh, qq, n0 + lane, p, d0);
+                pair(bh, qq, n0 + 64 + lane, p, d1);
+                for (int j = 0; j < kBN && n0 + j < s.S; ++j) {
+                    if (CAUSAL && n0 + (j & ~31) > m0 + kBM - 1) break;  // keys no query of the step sees
+                    const float dj = __shfl(j < 64 ? d0 : d1, j & 63, 64);
+                    if (lane < s.E) t = fmaf(dj, kb[(int64_t)(n0 + j) * s.E + lane], t);
+                }
+                if (lane < s.E) a.dq_part[(slot0 + (int64_t)bh * (s.L - rf) + (qq - rf)) * s.E + lane] = t;
+            }
+            if (kw0 >= s.S || (CAUSAL && m0 + kBM - 1 < kw0)) continue;
+            float p, ds;
+            pair(bh, qq, kw0 + lr, p, ds);
+            const float *x = static_cast<const float *>(values ? a.dout : a.q) + row * s.E;
+            const float w = values ? p : ds;
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int d = 32 * dt + acc_row(r, g);
+                    if (d < s.E) acc[dt][r] = fmaf(w, x[d], acc[dt][r]);
+                }
+        }
+    }
+}
+
+// key_tile on the bf16 matrix cores (x3.hpp), for head dims up to 64: the same tile, steps and
+// slots, eight waves in two groups that ping-pong.  Waves w and w + 4 share a SIMD and the same 32
+// keys; wave w (group A) forms S, P and dV, wave w + 4 (group B) dP, dS, dK and dQ:
+//
+//   phase 1 of step i   A: P(i), split, to LDS; stages dO(i + 1)     B: dQ, dK of i - 1, dP(i)  (MFMA)
+//   phase 2             A: dV(i), S(i + 1)                 (MFMA)    B: dS(i), split; stages Q(i + 2)
+//
+// with a barrier after each, so that in every phase one wave of a SIMD feeds the matrix cores (72
+// MFMAs in phase 1, 48 in phase 2 at D = 64) while the other has the VALU.  A wave alone does not
+// overlap the two well: an MFMA holds its wave's issue for half of its own time, and a dependent
+// VALU instruction waits 8 cycles.  (All of it in each of four waves, one per SIMD at 512 registers,
+// S and dP of the next step between the VALU work of this one: B8 H16 L1024 D64 full 681 us,
+// 35% of the matrix cores' time; this: 530 us, 46%.  On float32 MFMAs, with dS
+// shared by four waves through LDS: 655 us.  Issue priorities for the MFMA phases, or dQ in group A:
+// no faster, 2% slower.)
+//
+//   * K (A), V and K^T (B) of the wave's keys are split once and stay in registers; Q and dO are
+//     split on their way into LDS (three buffers of Q: S reads one ahead, dK one behind);
+//   * P goes from A to B in the accumulators' own layout; dS goes through B's own LDS tile to be
+//     read back with queries on lanes, so that each wave forms its 32 keys' share of dQ; the four
+//     shares are added in wave order through LDS, one phase later;
+//   * S takes the forward's products in the forward's order, so P = exp(S - lse) normalizes
+//     exactly as the forward's did.
+constexpr int kX3Threads = 2 * kThreads;
+
+template <int D>
+struct alignas(16) BwdSmemX3 {
+    X3Tile<kBM, D> q[3], o[2];       // at a tile's start the K, then V rows of the first four waves' keys
+    float p[kWaves][16][64];         // P, accumulator registers by lane
+    X3Tile<32, 32> ds[kWaves];       // dS: rows are keys, columns the step's queries
+    float part[kWaves][kBM][D + 4];  // a wave's share of dQ
+    float lse[2][kBM], dsum[2][kBM];
+    int open[kWaves];                // row masks: the wave's keys have one that is not -inf
+};
+
+// MASK: 0 none, 1 a value per (query, key), 2 the same for every query (key padding).
+template <int D, bool CAUSAL, int MASK, bool VEC>
+DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int kt, int i0, int i1, float *kdst,
+                      float *vdst, bool kv_atomic) {
+    constexpr int KSTEP = D / 16, NDT = D / 32;
+    const AttnShape &s = a.s;
+    const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3;
+    const bool group_a = wave8 < 4;
+    const int lane = tid & 63, lr = lane & 31, g = lane >> 5, gtid = tid & (kThreads - 1);
+    const int b = bhk / s.Hkv, hk = bhk % s.Hkv;
+    const int n0 = kt * kBN;
+    const int kw0 = n0 + wave * 32;  // this wave's first key
+    const int key = kw0 + lr;        // this lane's key column
+    const uint32_t rowb = row_lanebase<kBM, D>(lane), trb = tr_lanebase<kBM, D>(lane);
+    const float *mbase = MASK ? s.mask + (int64_t)b * s.msb : nullptr;
+
+    // Steps as (query head, first query), advanced without divisions.
+    const int m_begin = tile_m_begin(CAUSAL, kt), per_head = tile_per_head(s, kt);
+    struct Pos {
+        int bh, m0;
+    };
+    auto next_pos = [&](Pos p) {
+        p.m0 += kBM;
+        if (p.m0 >= s.L) p.m0 = m_begin, ++p.bh;
+        return p;
+    };
+    const bool dq_atomic = a.dq_part == nullptr;
+    const int rf = slot_from(s, kt);
+    const int64_t slot0 = slot_before(s, kt) * ((int64_t)s.B * s.H);
+    auto dq_dst = [&](Pos p) -> float * {
+        if (dq_atomic) return a.dq_acc + ((int64_t)p.bh * s.L + p.m0) * s.E;
+        return a.dq_part + (slot0 + (int64_t)p.bh * (s.L - rf) + (p.m0 - rf)) * s.E;
+    };
+    // Padding: a wave none of whose keys is visible to any query does no work (masks that differ
+    // between heads are not looked at).
+    int open = 15;
+    if (MASK == 2 && s.msh == 0) {
+        __syncthreads();  // a previous tile's last readers of sm.open are done
+        if (group_a) {
+            const bool any = __any(key < s.S && mbase[min(key, s.S - 1)] != -INFINITY);
+            if (lane == 0) sm.open[wave] = any;
+        }
+        __syncthreads();
+        open = __builtin_amdgcn_readfirstlane(sm.open[0] | sm.open[1] << 1 | sm.open[2] << 2 | sm.open[3] << 3);
+    }
+    // Wave w works in a step if some query of the step sees one of its keys.
+    auto live_at = [&](int w, int m0) {
+        return ((open >> w) & 1) && n0 + 32 * w < s.S && (!CAUSAL || m0 + kBM - 1 >= n0 + 32 * w);
+    };
+
+    f32x16 acc[NDT];  // dV^T (group A) or dK^T (group B) of this lane's key
+#pragma unroll
+    for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+    const Pos first{b * s.H + hk * s.repeat + (i0 < i1 ? i0 / per_head : 0), m_begin + (i0 < i1 ? i0 % per_head : 0) * kBM};
+
+    // The waves' shares of the dQ of the step at p, added and stored (or added into dq).
+    auto reduce_dq = [&](Pos p) {
+        float *dst = dq_dst(p);
+        const int rows = min(kBM, s.L - p.m0);
+        const int r = tid / (D / 4), d = tid % (D / 4) * 4;
+        if (kBM * D / 4 < kX3Threads && tid >= kBM * D / 4) return;
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+            if (live_at(w, p.m0)) t += *reinterpret_cast<const f32x4 *>(&sm.part[w][r][d]);
+        if (r >= rows) return;
+        if (!dq_atomic && (s.E & 3) == 0) {  // slots start 16-byte aligned and rows are whole parts
+            if (d < s.E) *reinterpret_cast<f32x4 *>(dst + (int64_t)r * s.E + d) = t;
+            return;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (d + e < s.E) {
+                if (dq_atomic) unsafeAtomicAdd(dst + (int64_t)r * s.E + d + e, t[e] * s.scale);
+                else dst[(int64_t)r * s.E + d + e] = t[e];
+            }
+    };
+
+    if (i0 < i1 && open == 0) {  // nothing visible: the tile's dQ shares are zero
+        if (!dq_atomic) {
+            Pos p = first;
+            for (int i = i0; i < i1; ++i, p = next_pos(p)) {
+                float *dst = dq_dst(p);
+                const int count = min(kBM, s.L - p.m0) * s.E;
+                for (int j = tid; j < count; j += kX3Threads) dst[j] = 0.f;
+            }
+        }
+    } else if (i0 < i1) {
+        // Group A stages dO (with lse and dsum), group B Q: a step at a time, in registers until the
+        // buffer it goes to is free.
+        X3Stage<kBM, D, kThreads, VEC> stage;
+        float lse_next = 0.f, dsum_next = 0.f;
+        Pos load_pos = first;
+        const float *sbase = static_cast<const float *>(group_a ? a.dout : a.q);
+        auto load_step = [&]() {
+            stage.load(sbase + (int64_t)load_pos.bh * s.L * s.E, load_pos.m0, s.L - 1, s.E, gtid);
+            if (group_a) {  // every thread its row modulo 32; queries past L: lse +inf, so P = 0
+                const int qq = load_pos.m0 + (gtid & (kBM - 1));
+                const int64_t at = (int64_t)load_pos.bh * s.L + min(qq, s.L - 1);
+                lse_next = qq < s.L ? a.lse[at] : INFINITY;
+                dsum_next = qq < s.L ? a.dsum[at] : 0.f;
+            }
+            load_pos = next_pos(load_pos);
+        };
+        auto store_do = [&](int buf) {
+            stage.store(sm.o[buf], gtid);
+            sm.lse[buf][gtid & (kBM - 1)] = lse_next, sm.dsum[buf][gtid & (kBM - 1)] = dsum_next;
+        };
+        // The keys' rows, through LDS tiles (waves w and w + 4 share tile w): K as A's row operand and
+        // B's transposed one, then V as B's row operand.
+        X3 kv[KSTEP], kT[NDT][2];
+        {
+            X3Tile<kBM, D> &wt = wave < 3 ? sm.q[wave] : sm.o[0];
+            X3Stage<kBM, D, 64, VEC> rows;
+            rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, lane);
+            load_step();
+            __syncthreads();  // a previous tile's last readers of these areas are done
+            if (group_a) rows.store(wt, lane);
+            __syncthreads();
+            if (group_a) {
+#pragma unroll
+                for (int st = 0; st < KSTEP; ++st) kv[st] = row_frag_x3(wt, rowb, 0, st);
+            } else {
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) kT[dt][u] = tr_frag_x3(wt, trb, 16 * u, dt);
+            }
+            __syncthreads();
+            if (!group_a) {
+                rows.store(wt, lane);
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int st = 0; st < KSTEP; ++st) kv[st] = row_frag_x3(wt, rowb, 0, st);
+            }
+            __syncthreads();
+        }
+        if (group_a) {
+            store_do(0);
+            if (i0 + 1 < i1) load_step();
+        } else {
+            stage.store(sm.q[0], gtid);
+            if (i0 + 1 < i1) {
+                load_step();
+                stage.store(sm.q[1], gtid);
+                if (i0 + 2 < i1) load_step();
+            }
+        }
+        __syncthreads();  // Q of the first two steps, dO of the first
+
+        Pos pos = first, prev{-1, 0};
+        bool live = live_at(wave, pos.m0);
+        if (group_a) {
+            float mrow = 0.f;
+            int mrow_bh = -1;
+            float mfull[MASK == 1 ? 16 : 1];
+            auto full_mask = [&](Pos p) {  // the mask of the step at p
+                if constexpr (MASK == 1) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int qq = p.m0 + acc_row(r, g);
+                        mfull[r] = (qq < s.L && key < s.S) ? mbase[(int64_t)(p.bh - b * s.H) * s.msh + (int64_t)qq * s.msl + key] : 0.f;
+                    }
+                }
+            };
+            f32x16 sacc;
+            X3 p3[2];
+            // S = Q K^T (queries are rows, the wave's keys columns), in k-step groups; and dV += P^T dO,
+            // in groups of 32 dims by 16 queries.
+            auto score_group = [&](int st, const X3 &q) {
+                if (st == 0) {
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+                }
+                sacc = mfma_x3_small_ba(q, kv[st], sacc);
+            };
+            auto score_rest = [&](int buf) {
+#pragma unroll
+                for (int st = 0; st < KSTEP; ++st)
+                    sacc = mfma_bf16(row_frag<kBM, D>(sm.q[buf].p[0], rowb, 0, st), kv[st].h, sacc);
+            };
+            auto value_group = [&](int gi, const X3 &o) { acc[gi % NDT] = mfma_x3(o, p3[gi / NDT], acc[gi % NDT]); };
+            auto scores = [&](int buf) {
+                pipelined<KSTEP>([&](int st) { return row_frag_x3(sm.q[buf], rowb, 0, st); }, score_group);
+                score_rest(buf);
+            };
+            if (live) {
+                full_mask(pos);
+                scores(0);
+            }
+            int qb = 0;  // buffer of Q(i)
+            for (int i = i0; i < i1; ++i) {
+                const Pos npos = next_pos(pos);
+                const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
+                const int ob = (i - i0) & 1;
+                qb = qb == 2 ? 0 : qb + 1;  // of Q(i + 1)
+                if (live) {
+                    if (MASK == 2 && pos.bh != mrow_bh) {
+                        mrow = key < s.S ? mbase[(int64_t)(pos.bh - b * s.H) * s.msh + key] : 0.f;
+                        mrow_bh = pos.bh;
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const f32x4 l4 = *reinterpret_cast<const f32x4 *>(&sm.lse[ob][8 * j + 4 * g]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            // scale * q.k (+ mask) - lse in natural-log units, as the reference forms
+                            // it, then one conversion to base 2 for v_exp_f32.
+                            const int r = 4 * j + e;
+                            float x = sacc[r] * s.scale;
+                            if (MASK == 1) x += mfull[MASK == 1 ? r : 0];
+                            if (MASK == 2) x += mrow;
+                            sacc[r] = exp2_fast((x - l4[e]) * kLog2e);
+                        }
+                    }
+                    // Keys past the end or (causal) past a query only occur when the wave's keys reach
+                    // the end of the sequence or cross the diagonal of this query tile.
+                    if (kw0 + 31 >= s.S || (CAUSAL && kw0 + 31 > pos.m0)) {
+                        asm volatile("" ::: "memory");  // keeps the branch: not if-converted into selects
+#pragma unroll
+                        for (int r = 0; r < 16; ++r)
+                            if (key >= s.S || (CAUSAL && key > pos.m0 + acc_row(r, g))) sacc[r] = 0.f;
+                    }
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sm.p[wave][r][lane] = sacc[r];
+                    p3[0] = split3(sacc, 0);
+                    p3[1] = split3(sacc, 8);
+                }
+                if (i + 1 < i1) {
+                    store_do(ob ^ 1);
+                    if (i + 2 < i1) load_step();
+                }
+                __syncthreads();
+                if (nlive) full_mask(npos);
+                auto read_do = [&](int gi) { return tr_frag_x3(sm.o[ob], trb, 16 * (gi / NDT), gi % NDT); };
+                if (live && nlive) {
+                    pipelined<2 * NDT + KSTEP>(
+                        [&](int k) { return k < 2 * NDT ? read_do(k) : row_frag_x3(sm.q[qb], rowb, 0, k - 2 * NDT); },
+                        [&](int k, const X3 &f) {
+                            if (k < 2 * NDT) value_group(k, f);
+                            else score_group(k - 2 * NDT, f);
+                        });
+                    score_rest(qb);
+                } else {
+                    if (live) pipelined<2 * NDT>(read_do, value_group);
+                    if (nlive) scores(qb);
+                }
+                if (prev.bh >= 0) reduce_dq(prev);
+                live = nlive;
+                prev = pos, pos = npos;
+                __syncthreads();
+            }
+            __syncthreads();
+        } else {
+            const uint32_t dstrb = tr_lanebase<32, 32>(lane);
+            f32x16 pacc;
+            X3 d3[2];
+            auto dq_share = [&]() {  // of the step whose dS is in the wave's tile
+                const X3 dsT[2] = {tr_frag_x3(sm.ds[wave], dstrb, 0, 0), tr_frag_x3(sm.ds[wave], dstrb, 16, 0)};
+#pragma unroll
+                for (int dt = 0; dt < NDT; ++dt) {
+                    f32x16 dq;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) dq[r] = 0.f;
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) dq = mfma_x3(kT[dt][u], dsT[u], dq);
+#pragma unroll
+                    for (int r = 0; r < 16; r += 4)
+                        *reinterpret_cast<f32x4 *>(&sm.part[wave][lr][32 * dt + acc_row(r, g)]) =
+                            f32x4{dq[r], dq[r + 1], dq[r + 2], dq[r + 3]};
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            };
+            auto key_group = [&](int gi, const X3 &q) { acc[gi % NDT] = mfma_x3(q, d3[gi / NDT], acc[gi % NDT]); };
+            auto prob_group = [&](int st, const X3 &o) { pacc = mfma_x3(o, kv[st], pacc); };
+            int pb = 2;  // buffer of Q(i - 1)
+            bool plive = false;
+            for (int i = i0; i < i1; ++i) {
+                const Pos npos = next_pos(pos);
+                const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
+                const int ob = (i - i0) & 1;
+                // dK += dS^T Q of the step before, and dP = dO V^T.
+                auto read_q = [&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); };
+                auto read_do = [&](int st) { return row_frag_x3(sm.o[ob], rowb, 0, st); };
+                if (plive) dq_share();
+#pragma unroll
+                for (int r = 0; r < 16; ++r) pacc[r] = 0.f;
+                if (plive && live) {
+                    pipelined<2 * NDT + KSTEP>([&](int k) { return k < 2 * NDT ? read_q(k) : read_do(k - 2 * NDT); },
+                                               [&](int k, const X3 &f) {
+                                                   if (k < 2 * NDT) key_group(k, f);
+                                                   else prob_group(k - 2 * NDT, f);
+                                               });
+                } else {
+                    if (plive) pipelined<2 * NDT>(read_q, key_group);
+                    if (live) pipelined<KSTEP>(read_do, prob_group);
+                }
+                __syncthreads();
+                if (live) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&sm.dsum[ob][8 * j + 4 * g]);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int r = 4 * j + e;
+                            pacc[r] = sm.p[wave][r][lane] * (pacc[r] - d4[e]);
+                        }
+                    }
+                    // Into the dS tile: rows are keys, columns queries (registers 8u .. 8u + 7 hold
+                    // queries 16u + 4g + 0..3 and 16u + 8 + 4g + 0..3).
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        d3[u] = split3(pacc, 8 * u);
+                        const bf16x8 parts[3] = {d3[u].h, d3[u].m, d3[u].l};
+#pragma unroll
+                        for (int pl = 0; pl < 3; ++pl) {
+                            const u32x4 w = __builtin_bit_cast(u32x4, parts[pl]);
+                            uint32_t *row = reinterpret_cast<uint32_t *>(&sm.ds[wave].p[pl][2 * u * CMTile<32, 32>::P + lr]) + 2 * g;
+                            *reinterpret_cast<uint64_t *>(row) = (uint64_t)w[0] | ((uint64_t)w[1] << 32);
+                            *reinterpret_cast<uint64_t *>(row + CMTile<32, 32>::P * 4) = (uint64_t)w[2] | ((uint64_t)w[3] << 32);
+                        }
+                    }
+                }
+                if (prev.bh >= 0) reduce_dq(prev);
+                if (i + 2 < i1) {
+                    stage.store(sm.q[pb], gtid);  // Q(i + 2) where Q(i - 1) was
+                    if (i + 3 < i1) load_step();
+                }
+                pb = pb == 2 ? 0 : pb + 1;
+                plive = live, live = nlive;
+                prev = pos, pos = npos;
+                __syncthreads();
+            }
+            if (plive) {
+                dq_share();
+                pipelined<2 * NDT>([&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); }, key_group);
+            }
+            __syncthreads();
+        }
+        reduce_dq(prev);
+
+        // Not finite: the tile's steps again in plain float32 (x3.hpp).
+        float bad = 0.f;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt) bad += not_finite(acc[dt]);
+        if (__syncthreads_or(bad != 0.f)) redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+    }
+
+    // dV, or dK times scale, of this lane's key.
+    const float mul = group_a ? 1.f : s.scale;
+    float *tile_dst = group_a ? vdst : kdst;
+    if (kv_atomic) {
+        // A share of the tile's steps, added atomically through LDS: one atomic instruction then
+        // covers consecutive dims of one key (see key_tile).
+        constexpr int RS = D + 4;
+        static_assert(2 * kWaves * 32 * RS * sizeof(float) <= sizeof(BwdSmemX3<D>), "per-wave blocks fit");
+        float *blk = reinterpret_cast<float *>(&sm) + wave8 * 32 * RS;
+        const int rows = min(32, s.S - kw0);
+        __syncthreads();  // the previous readers of the area are done
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4)
+                *reinterpret_cast<f32x4 *>(blk + lr * RS + dt * 32 + acc_row(r, g)) =
+                    f32x4{acc[dt][r] * mul, acc[dt][r + 1] * mul, acc[dt][r + 2] * mul, acc[dt][r + 3] * mul};
+        __syncthreads();
+        float *dst = tile_dst + (int64_t)(kw0 - n0) * s.E;
+        for (int i = lane; i < rows * D; i += 64) {
+            const int rr = i / D, d = i % D;
+            if (d < s.E) unsafeAtomicAdd(dst + (int64_t)rr * s.E + d, blk[rr * RS + d]);
+        }
+        return;
+    }
+    if (key < s.S) {
+        float *dst = tile_dst + (int64_t)(key - n0) * s.E;
+#pragma unroll
+        for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+            for (int r = 0; r < 16; r += 4) {
+                const int d = dt * 32 + acc_row(r, g);
+                if (VEC) {
+                    if (d < s.E)
+                        *reinterpret_cast<f32x4 *>(dst + d) =
+                            f32x4{acc[dt][r] * mul, acc[dt][r + 1] * mul, acc[dt][r + 2] * mul, acc[dt][r + 3] * mul};
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (d + u < s.E) dst[d + u] = acc[dt][r + u] * mul;
+                }
+            }
+    }
+}
+
 // key_tile at D = 128: 8 waves of 16 keys (v_mfma_f32_16x16x4_f32), two waves per SIMD.  With 32
 // keys per wave (key_tile) the dK^T, dV^T accumulators and the V row take ~290 registers of a
 // wave, so that kernel ran one wave per SIMD; here each wave holds 2 x 32 accumulator registers
@@ -520,8 +1007,7 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
 // with the forward's product and pairing of dims (v_mfma_f32_32x32x2_f32), so P = exp(S - lse)
 // normalizes to the forward's lse exactly; here S is rounded in another order, ~1e-5 relative
 // apart for scores near 100 (gradient errors up to ~5x the oracle's there; at ordinary scores
-// far below the bar).  The same layout at D = 64 measured 355 -> 343 us on B8 H12 L1024 but
-// keeps key_tile for that consistency.  The products:
+// far below the bar).  The products:
 //   * S and dP with queries as rows, in two 16-query halves: the reduction over d runs in 16-dim
 //     blocks whose step u gives lane l dim 16 j + 4 (l / 16) + u, so a lane's Q and dO operands
 //     for a block are one ds_read_b128 each, its V operands registers and its K operands four
@@ -532,7 +1018,6 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
 template <int D, bool CAUSAL, bool MASK, bool VEC>
 DEVI void key_tile16(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, int i0, int i1, float *kdst,
                      float *vdst, bool kv_atomic) {
-    static_assert(kSixteenKeys(D), "the 8-wave tile is for head dim 128");
     constexpr int NT = 2 * kThreads, NKB = D / 16;
 
     const AttnShape &s = a.s;
@@ -784,8 +1269,8 @@ DEVI void key_tile_any(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int k
         key_tile<D, CAUSAL, MASK, VEC>(a, sm, tid, bhk, kt, i0, i1, kdst, vdst, kv_atomic);
 }
 
-template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16 = kSixteenKeys(D)>
-__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(D, MASK, K16), bwd_waves_per_eu(D, MASK, K16)))) void bwd_f32_kernel(BwdArgs a) {
+template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16>
+__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(K16), bwd_waves_per_eu(K16)))) void bwd_f32_kernel(BwdArgs a) {
     __shared__ BwdSmem<D> sm;
     const int BHk = a.s.B * a.s.Hkv;
     const int kt = blockIdx.x / BHk;  // tile 0 has the most causal work, so it goes first
@@ -793,6 +1278,17 @@ __global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_pe
     const int64_t row0 = ((int64_t)bhk * a.s.S + (int64_t)kt * kBN) * a.s.E;
     key_tile_any<D, CAUSAL, MASK, VEC, K16>(a, sm, threadIdx.x, bhk, kt, 0, tile_steps(a.s, kt),
                                    static_cast<float *>(a.dk) + row0, static_cast<float *>(a.dv) + row0, false);
+}
+
+template <int D, bool CAUSAL, int MASK, bool VEC>
+__global__ __launch_bounds__(kX3Threads) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_x3_kernel(BwdArgs a) {
+    __shared__ BwdSmemX3<D> sm;
+    const int BHk = a.s.B * a.s.Hkv;
+    const int kt = blockIdx.x / BHk;  // tile 0 has the most causal work, so it goes first
+    const int bhk = blockIdx.x % BHk;
+    const int64_t row0 = ((int64_t)bhk * a.s.S + (int64_t)kt * kBN) * a.s.E;
+    key_tile_x3<D, CAUSAL, MASK, VEC>(a, sm, threadIdx.x, bhk, kt, 0, tile_steps(a.s, kt),
+                                      static_cast<float *>(a.dk) + row0, static_cast<float *>(a.dv) + row0, false);
 }
 
 // Where a stream-K range's share of a key tile it cuts goes: slot 0 of the range for the tile it
@@ -804,10 +1300,9 @@ DEVI float *kv_slot(const BwdArgs &a, int64_t range, int which) {
 
 // One workgroup per range of the stream-K schedule, ranges dealt to the 8 XCDs in contiguous
 // blocks (workgroup w runs on XCD w % 8), so the key tiles of one kv head, which read the same
-// Q / dO, share an L2.
-template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16 = kSixteenKeys(D)>
-__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(D, MASK, K16), bwd_waves_per_eu(D, MASK, K16)))) void bwd_f32_streamk_kernel(BwdArgs a, StreamK sk) {
-    __shared__ BwdSmem<D> sm;
+// Q / dO, share an L2.  tile(bhk, kt, i0, i1, kdst, vdst, atomic) runs steps [i0, i1) of a key tile.
+template <typename F>
+DEVI void streamk_range(const BwdArgs &a, const StreamK &sk, F tile) {
     const int w = blockIdx.x;
     const int64_t c = (int64_t)(w & 7) * (sk.chunks >> 3) + (w >> 3);
     int64_t pos = c * sk.total / sk.chunks;
@@ -826,7 +1321,7 @@ __global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_pe
     while (pos < end) {
         const int n = tile_steps(a.s, kt);
         const int i1 = (int)min((int64_t)n, i + (end - pos));
-        if (!first) __syncthreads();  // the previous tile's last dQ product has read sm.kt, sm.ds
+        if (!first) __syncthreads();  // the previous tile's last readers of the shared area are done
         const bool whole = i == 0 && i1 == n;
         const int64_t row0 = ((int64_t)bhk * a.s.S + (int64_t)kt * kBN) * a.s.E;
         float *kd = static_cast<float *>(a.dk) + row0, *vd = static_cast<float *>(a.dv) + row0;
@@ -834,7 +1329,7 @@ __global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_pe
             kd = kv_slot(a, c, first ? 0 : 1);
             vd = kd + (int64_t)kBN * a.s.E;
         }
-        key_tile_any<D, CAUSAL, MASK, VEC, K16>(a, sm, threadIdx.x, bhk, kt, i, i1, kd, vd, !whole && !a.kv_part);
+        tile(bhk, kt, i, i1, kd, vd, !whole && !a.kv_part);
         first = false;
         pos += i1 - i;
         i = 0;
@@ -842,6 +1337,22 @@ __global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_pe
             if (++kt == nkt) kt = 0, ++bhk;
         } while (pos < end && tile_steps(a.s, kt) == 0);
     }
+}
+
+template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16>
+__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(K16), bwd_waves_per_eu(K16)))) void bwd_f32_streamk_kernel(BwdArgs a, StreamK sk) {
+    __shared__ BwdSmem<D> sm;
+    streamk_range(a, sk, [&](int bhk, int kt, int i0, int i1, float *kd, float *vd, bool atomic) {
+        key_tile_any<D, CAUSAL, MASK, VEC, K16>(a, sm, threadIdx.x, bhk, kt, i0, i1, kd, vd, atomic);
+    });
+}
+
+template <int D, bool CAUSAL, int MASK, bool VEC>
+__global__ __launch_bounds__(kX3Threads) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_x3_streamk_kernel(BwdArgs a, StreamK sk) {
+    __shared__ BwdSmemX3<D> sm;
+    streamk_range(a, sk, [&](int bhk, int kt, int i0, int i1, float *kd, float *vd, bool atomic) {
+        key_tile_x3<D, CAUSAL, MASK, VEC>(a, sm, threadIdx.x, bhk, kt, i0, i1, kd, vd, atomic);
+    });
 }
 
 // A key tile of the stream-K schedule: its first step's position and step count; `cut` when its
@@ -1014,28 +1525,51 @@ size_t dq_part_bytes(const AttnShape &s) {
 size_t kv_part_bytes(const StreamK &sk, int E) { return (size_t)sk.chunks * 4 * kBN * E * sizeof(float); }
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-template <int D, bool VEC, bool K16>
-hipError_t launch_dv(const BwdArgs &a, const StreamK &sk, hipStream_t st) {
-    const bool mask = a.s.mask != nullptr;
+// Head dims 65 to 128 (float32 MFMA): whole tiles or stream-K ranges.
+template <bool VEC, bool K16>
+hipError_t launch_128(const BwdArgs &a, const StreamK &sk, dim3 grid, hipStream_t st) {
+    const dim3 block(layout_threads(K16));
+    auto go = [&](auto causal, auto mask) {
+        constexpr bool C = decltype(causal)::value, M = decltype(mask)::value;
+        if (sk.chunks > 0) return launch(bwd_f32_streamk_kernel<128, C, M, VEC, K16>, grid, block, st, a, sk);
+        return launch(bwd_f32_kernel<128, C, M, VEC, K16>, grid, block, st, a);
+    };
+    const std::true_type yes;
+    const std::false_type no;
+    if (a.s.mask) return a.s.causal ? go(yes, yes) : go(no, yes);
+    return a.s.causal ? go(yes, no) : go(no, no);
+}
+
+// Head dims up to 64 (split products on the bf16 matrix cores).
+template <int D, int MASK, bool VEC>
+hipError_t launch_x3(const BwdArgs &a, const StreamK &sk, dim3 grid, hipStream_t st) {
+    const dim3 block(kX3Threads);
     if (sk.chunks > 0) {
-        const dim3 grid(sk.chunks), block(layout_threads(K16));
-        if (a.s.causal && mask) return launch(bwd_f32_streamk_kernel<D, true, true, VEC, K16>, grid, block, st, a, sk);
-        if (a.s.causal) return launch(bwd_f32_streamk_kernel<D, true, false, VEC, K16>, grid, block, st, a, sk);
-        if (mask) return launch(bwd_f32_streamk_kernel<D, false, true, VEC, K16>, grid, block, st, a, sk);
-        return launch(bwd_f32_streamk_kernel<D, false, false, VEC, K16>, grid, block, st, a, sk);
+        if (a.s.causal) return launch(bwd_x3_streamk_kernel<D, true, MASK, VEC>, grid, block, st, a, sk);
+        return launch(bwd_x3_streamk_kernel<D, false, MASK, VEC>, grid, block, st, a, sk);
     }
+    if (a.s.causal) return launch(bwd_x3_kernel<D, true, MASK, VEC>, grid, block, st, a);
+    return launch(bwd_x3_kernel<D, false, MASK, VEC>, grid, block, st, a);
+}
+
+template <int D, bool VEC>
+hipError_t launch_tiles(const BwdArgs &a, const StreamK &sk, hipStream_t st) {
     const int nkt = (a.s.S + kBN - 1) / kBN;
-    const dim3 grid(nkt * a.s.B * a.s.Hkv), block(layout_threads(K16));
-    if (a.s.causal && mask) return launch(bwd_f32_kernel<D, true, true, VEC, K16>, grid, block, st, a);
-    if (a.s.causal) return launch(bwd_f32_kernel<D, true, false, VEC, K16>, grid, block, st, a);
-    if (mask) return launch(bwd_f32_kernel<D, false, true, VEC, K16>, grid, block, st, a);
-    return launch(bwd_f32_kernel<D, false, false, VEC, K16>, grid, block, st, a);
+    const dim3 grid(sk.chunks > 0 ? sk.chunks : nkt * a.s.B * a.s.Hkv);
+    if constexpr (D == 128) {  // the 8-wave tile of 16 keys, or on request the forward-consistent 4-wave tile
+        return a.s.consistent ? launch_128<VEC, false>(a, sk, grid, st) : launch_128<VEC, true>(a, sk, grid, st);
+    } else {
+        if (!a.s.mask) return launch_x3<D, 0, VEC>(a, sk, grid, st);
+        return a.s.msl == 0 ? launch_x3<D, 2, VEC>(a, sk, grid, st) : launch_x3<D, 1, VEC>(a, sk, grid, st);
+    }
 }
 
 template <int D>
 hipError_t launch_d(const BwdArgs &args, size_t part_bytes, hipStream_t st) {
     BwdArgs a = args;
-    a.s.vec = args.s.vec && args.s.E == D;  // the ABI checked 16-byte alignment; E must fill D
+    // The ABI checked 16-byte alignment; the float32 tiles want E to fill D, the others whole
+    // 16-byte parts of rows.
+    a.s.vec = args.s.vec && (D == 128 ? args.s.E == D : args.s.E % 4 == 0);
     const StreamK sk = plan_streamk(a.s, D, a.s.mask != nullptr);
     record_schedule(streamk_ranges, sk.chunks);
     // Deterministic when the workspace holds the slots; otherwise float atomics.
@@ -1053,12 +1587,7 @@ hipError_t launch_d(const BwdArgs &args, size_t part_bytes, hipStream_t st) {
     if (rows_blocks + zero_blocks > 0)
         return_if(launch(bwd_pre_f32_kernel, dim3((unsigned)(rows_blocks + zero_blocks)), dim3(256), st, a, sk,
                          rows_blocks));
-    // D = 128: the 8-wave tile of 16 keys, or on request the forward-consistent 4-wave tile.
-    if (D == 128 && a.s.consistent)
-        return_if((a.s.vec ? launch_dv<D, true, false>(a, sk, st) : launch_dv<D, false, false>(a, sk, st)));
-    else
-        return_if((a.s.vec ? launch_dv<D, true, kSixteenKeys(D)>(a, sk, st)
-                           : launch_dv<D, false, kSixteenKeys(D)>(a, sk, st)));
+    return_if((a.s.vec ? launch_tiles<D, true>(a, sk, st) : launch_tiles<D, false>(a, sk, st)));
     if (!a.dq_part) return hipSuccess;
     const int64_t dq_threads = rows * ((a.s.E + 3) / 4);
     const int dq_blocks = (int)((dq_threads + 255) / 256);

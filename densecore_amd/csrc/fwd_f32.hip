@@ -1,4 +1,5 @@
-// Float32 attention forward on CDNA4 MFMA (v_mfma_f32_32x32x2_f32).
+// Float32 attention forward on CDNA4's float32 MFMA (v_mfma_f32_32x32x2_f32), for head dim 128
+// (fwd_x3.hip: smaller ones), and the choice between the two.
 //
 // Computes what DenseCore's torch_attention::forward computes (src/torch_attention.rs:143-284):
 // out = softmax(scale * q k^T + mask, causal) v and lse = max + ln(sum), with fully masked
@@ -20,13 +21,12 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "fwd_order.hpp"
 #include "fwd_split.hpp"
 #include "params.hpp"
 
 namespace dc {
 namespace {
-
-// W waves per workgroup, 32 queries per wave (4; 2 or 1 for short causal problems).
 
 template <int D, int BN>
 struct alignas(16) FwdSmem {
@@ -97,14 +97,9 @@ DEVI int swz(int row) {
     return (row ^ ((row & 4) << 1)) & (D / 4 - 1);
 }
 
-// Global loads per wave for one K (or V) tile: each wave-wide load fills 64 / (D / 4) rows.
-template <int D, int BN, int W>
-constexpr int kTileLoads = BN / W / (64 / (D / 4));
-
-// Issue this wave's share of tile [n0, n0 + BN) into buffer `buf`: K and V, or only one of
-// them (keys past the end read a valid row, S - 1; their scores are -inf, so they contribute
+// Issue this wave's share of tile [n0, n0 + BN) (keys past the end read a valid row, S - 1; their scores are -inf, so they contribute
 // nothing).
-template <int D, int BN, int W, bool DO_K = true, bool DO_V = true>
+template <int D, int BN, int W>
 DEVI void issue_tile(FwdSmemAsync<D, BN> &sm, const float *kb, const float *vb, int n0, int S,
                      int wave, int lane) {
     constexpr int C = D / 4;             // 16-byte chunks per row
@@ -122,27 +117,12 @@ DEVI void issue_tile(FwdSmemAsync<D, BN> &sm, const float *kb, const float *vb, 
             const int row = wave * ROWS + j * RPL + lane / C;
             return (uint32_t)(row * D + (((lane % C) ^ swz<D>(row)) << 2)) * 4u;
         };
-        if constexpr (W == 1 && (DO_K != DO_V)) {
-            // One-wave workgroups (K or V alone): transfers in pairs, one m0 save per pair and the
-            // LDS address cast once (B64 H6 L256 causal 41.4 -> 40.5 us; the 4-wave kernels, whose
-            // wave index the LDS addresses carry, measured ~1% slower this way).
-            const uint64_t gb = sgpr_addr(DO_K ? kt : vt);
-            const uint32_t lb = lds_addr(DO_K ? &sm.k[0][0] : &sm.v[0][0]);
-#pragma unroll
-            for (int j = 0; j + 1 < NJ; j += 2)
-                lds_dma16_pair(gb, lane_off(j), lb + (uint32_t)(j * RPL * D * 4), gb, lane_off(j + 1),
-                               lb + (uint32_t)((j + 1) * RPL * D * 4));
-            if constexpr (NJ % 2 == 1)
-                lds_dma16_off(DO_K ? kt : vt, lane_off(NJ - 1),
-                              DO_K ? &sm.k[(NJ - 1) * RPL][0] : &sm.v[(NJ - 1) * RPL][0]);
-            return;
-        }
 #pragma unroll
         for (int j = 0; j < NJ; ++j) {
             const int r0 = wave * ROWS + j * RPL;
             const uint32_t off = lane_off(j);
-            if constexpr (DO_K) lds_dma16_off(kt, off, &sm.k[r0][0]);
-            if constexpr (DO_V) lds_dma16_off(vt, off, &sm.v[r0][0]);
+            lds_dma16_off(kt, off, &sm.k[r0][0]);
+            lds_dma16_off(vt, off, &sm.v[r0][0]);
         }
         return;
     }
@@ -152,27 +132,19 @@ DEVI void issue_tile(FwdSmemAsync<D, BN> &sm, const float *kb, const float *vb, 
         const int row = r0 + lane / C;
         const int chunk = (lane % C) ^ swz<D>(row);  // logical chunk stored at this slot
         const int64_t off = (int64_t)min(n0 + row, S - 1) * D + chunk * 4;
-        if constexpr (DO_K) lds_dma16(kb + off, &sm.k[r0][0]);
-        if constexpr (DO_V) lds_dma16(vb + off, &sm.v[r0][0]);
+        lds_dma16(kb + off, &sm.k[r0][0]);
+        lds_dma16(vb + off, &sm.v[r0][0]);
     }
 }
 
 template <int D, int BN, int W, bool CAUSAL, bool MASK, bool ASYNC, bool ROWMASK = false, bool SPLIT = false>
-__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 || !ASYNC ? 2 : 1, D <= 64 || !ASYNC ? 2 : 1))) void fwd_f32_kernel(FwdArgs a) {
+__global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(!ASYNC ? 2 : 1, !ASYNC ? 2 : 1))) void fwd_f32_kernel(FwdArgs a) {
     [[maybe_unused]] constexpr int kThreads = 64 * W;
     constexpr int kBM = 32 * W;
     constexpr int NT = BN / 32;  // key sub-tiles of 32 per kv tile
     constexpr int DH = D / 2;    // head-dim values each half-wave supplies per query
-    // One-wave workgroups (short causal rows without a mask) stage K and V in ONE buffer,
-    // loaded out of phase: K(t + 1) streams in while the wave computes softmax(t) and P V(t),
-    // V(t + 1) while it computes Q K(t + 1).  16 KB of LDS per wave at D = 64 and no barriers:
-    // ten independent waves per CU, dispatched longest first.  (Two-wave workgroups couple
-    // their SIMDs through each tile's barrier, which left the long query tiles of such problems
-    // sharing their SIMDs for most of the kernel: B64 H6 L256 D64 47.0 -> 43.1 us.)
-    constexpr bool ONEBUF = ASYNC && W == 1 && !MASK && !SPLIT;
-    constexpr int NLD = kTileLoads<D, BN, W>;
     using Smem = typename std::conditional<ASYNC, FwdSmemAsync<D, BN>, FwdSmem<D, BN>>::type;
-    using Smem2 = typename std::conditional<ASYNC && !ONEBUF, FwdSmemAsync<D, BN>, NoSmem>::type;
+    using Smem2 = typename std::conditional<ASYNC, FwdSmemAsync<D, BN>, NoSmem>::type;
     __shared__ Smem sm;
     __shared__ Smem2 sm2;  // the second buffer of the asynchronous path
 
@@ -268,12 +240,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
     const int t_end = SPLIT ? (piece + 1) * ntiles / npieces : ntiles;
 
     KVStage<D, BN, W> stage;
-    if constexpr (ONEBUF) {
-        if (t_begin < t_end) {
-            issue_tile<D, BN, W, true, false>(sm, kb, vb, t_begin * BN, s.S, wave, lane);
-            issue_tile<D, BN, W, false, true>(sm, kb, vb, t_begin * BN, s.S, wave, lane);
-        }
-    } else if constexpr (ASYNC) {
+    if constexpr (ASYNC) {
         if (t_begin < t_end) issue_tile<D, BN, W>(sm, kb, vb, t_begin * BN, s.S, wave, lane);
     } else if (s.vec && t_begin < t_end) {
         stage.load(kb, vb, t_begin * BN, s.S, tid);
@@ -285,11 +252,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
     // tn: the tile to stream in next (t + 1; -1: none).
     auto tile = [&](int t, auto &cur, auto &nxt, int tn) {
         const int n0 = t * BN;
-        if constexpr (ONEBUF) {
-            // In flight: K(t), then V(t).  (Every tile of a one-buffer wave has visible keys:
-            // causal tiles end at the wave's last query, so no tile takes the early return.)
-            wait_vmem_but<NLD>();
-        } else if constexpr (ASYNC) {
+        if constexpr (ASYNC) {
             __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads of tile t landed
             __syncthreads();  // everyone's loads landed; everyone is done with the previous tile
             if (tn >= 0) issue_tile<D, BN, W>(nxt, kb, vb, tn * BN, s.S, wave, lane);
@@ -387,27 +350,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
             }
         }
 
-        if constexpr (ONEBUF) {
-            wait_lds();  // K(t)'s reads have returned: the buffer takes K(t + 1)
-            if (tn >= 0) issue_tile<D, BN, W, true, false>(sm, kb, vb, tn * BN, s.S, wave, lane);
-            // In flight: V(t), then K(t + 1).
-            if (tn >= 0) wait_vmem_but<NLD>();
-            else wait_vmem();
-        }
-        // With two or more waves the V operands are read ahead here (their LDS latency hides
-        // under the softmax) and each P column feeds its products as soon as it is formed:
-        // B8 H12 L1024 causal 131.4 -> 129.8 us, B1 H8 L2048 62.0 -> 60.1 us.  (One-wave
-        // workgroups measured faster without: 43.1 against 43.9 us.)
-        constexpr bool VAHEAD = D <= 64 && !ONEBUF;
-        float vv[VAHEAD ? NT : 1][VAHEAD ? D / 32 : 1][16];
-        if constexpr (VAHEAD) {
-#pragma unroll
-            for (int kt = 0; kt < NT; ++kt)
-#pragma unroll
-                for (int dt = 0; dt < D / 32; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) vv[kt][dt][r] = vread(kt * 32 + acc_row(r, g), dt * 32 + lr);
-        }
         // Scores in log2 units (with a mask; without one the raw products, see csc), masked on
         // edge tiles; tile max per query.
         // A row mask arrives times log2 e, so its score is one FMA with scale log2 e (bit-identical
@@ -457,21 +399,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
         }
         const float m_use = m_run == -INFINITY ? 0.f : m_run;
         float ls = 0.f;
-        if constexpr (VAHEAD) {
-#pragma unroll
-            for (int kt = 0; kt < NT; ++kt)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float p = expo(sacc[kt][r], m_use);
-                    ls += p;
-                    if (live[kt]) {
-#pragma unroll
-                        for (int dt = 0; dt < D / 32; ++dt) oacc[dt] = mfma_f32(vv[kt][dt][r], p, oacc[dt]);
-                    }
-                }
-            l_run += xor32_add(ls);
-            return;
-        }
 #pragma unroll
         for (int kt = 0; kt < NT; ++kt)
 #pragma unroll
@@ -494,15 +421,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
                                         oacc[dt]);
         }
     };
-    if constexpr (ONEBUF) {
-        wait_vmem();  // the queries (and tile t_begin): no load of the loop waits for them again
-        for (int t = t_begin; t < t_end; ++t) {
-            const int tn = t + 1 < t_end ? t + 1 : -1;
-            tile(t, sm, sm, tn);
-            wait_lds();  // V(t)'s reads have returned: the buffer takes V(t + 1)
-            if (tn >= 0) issue_tile<D, BN, W, false, true>(sm, kb, vb, tn * BN, s.S, wave, lane);
-        }
-    } else if constexpr (ASYNC) {
+    if constexpr (ASYNC) {
         for (int t = t_begin; t < t_end; t += 2) {
             tile(t, sm, sm2, t + 1 < t_end ? t + 1 : -1);
             if (t + 1 < t_end) tile(t + 1, sm2, sm, t + 2 < t_end ? t + 2 : -1);
@@ -544,95 +463,6 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(D <= 64 
     }
 }
 
-// The BN-key tiles of one mask row (S keys) that hold any key whose mask is not -inf, counted by
-// one wave.  The loads of 8 x 64 keys are all issued before any is tested, so a row costs one
-// memory latency per 512 keys instead of one per 64 (C3's step, order pass plus forward: 90.7 ->
-// 90.4 us; the rest of the pass is its launch).
-template <int BN>
-DEVI int live_tiles(const float *row, int S, int lane) {
-    constexpr int U = 8;
-    int c = 0;
-    for (int k0 = 0; k0 < S; k0 += 64 * U) {
-        float x[U];
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int key = k0 + 64 * u + lane;
-            x[u] = key < S ? row[key] : -INFINITY;
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const uint64_t live = __ballot(x[u] != -INFINITY);
-            if (BN == 64) c += live != 0;
-            else c += ((live & 0xffffffffull) != 0) + ((live >> 32) != 0);
-        }
-    }
-    return c;
-}
-
-// One wave per (b, h) of a query-independent mask: the number of BN-key tiles that hold any key
-// whose mask is not -inf (the tiles the forward computes; the others it skips).
-template <int BN>
-__global__ __launch_bounds__(64) void rowmask_tiles_kernel(FwdArgs a) {
-    static_assert(BN == 32 || BN == 64, "one or two tiles per wave-wide pass");
-    const AttnShape &s = a.s;
-    const int bh = blockIdx.x, lane = threadIdx.x;
-    const float *row = s.mask + (int64_t)(bh / s.H) * s.msb + (int64_t)(bh % s.H) * s.msh;
-    const int count = live_tiles<BN>(row, s.S, lane);
-    if (lane == 0) a.tiles[bh] = count;
-}
-
-// One workgroup: a counting sort of the heads by live tiles, descending (ties in any order; the
-// results do not depend on the order).
-__global__ __launch_bounds__(1024) void rowmask_order_kernel(FwdArgs a, int ntiles) {
-    __shared__ int start[kOrderMaxTiles + 1];
-    const int BH = a.s.B * a.s.H, tid = threadIdx.x;
-    for (int v = tid; v <= ntiles; v += 1024) start[v] = 0;
-    __syncthreads();
-    for (int i = tid; i < BH; i += 1024) atomicAdd(&start[a.tiles[i]], 1);
-    __syncthreads();
-    if (tid == 0) {  // start[v] = number of heads with more live tiles than v
-        int run = 0;
-        for (int v = ntiles; v >= 0; --v) {
-            const int c = start[v];
-            start[v] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    for (int i = tid; i < BH; i += 1024) a.order[atomicAdd(&start[a.tiles[i]], 1)] = i;
-}
-
-// Masks that depend on the batch and the key only (head and query strides 0: key padding, C3):
-// one launch instead of the two above.  One workgroup counts the live tiles of each batch's mask
-// row, a wave per row, and sorts the heads by their batch's count, descending.
-template <int BN>
-__global__ __launch_bounds__(1024) void rowmask_batch_order_kernel(FwdArgs a, int ntiles) {
-    static_assert(BN == 32 || BN == 64, "one or two tiles per wave-wide pass");
-    __shared__ int count[kOrderMaxBatch];
-    __shared__ int start[kOrderMaxTiles + 1];
-    const AttnShape &s = a.s;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int v = tid; v <= ntiles; v += 1024) start[v] = 0;
-    for (int b = wave; b < s.B; b += 16) {
-        const int c = live_tiles<BN>(s.mask + (int64_t)b * s.msb, s.S, lane);
-        if (lane == 0) count[b] = c;
-    }
-    __syncthreads();
-    const int BH = s.B * s.H;
-    for (int i = tid; i < BH; i += 1024) atomicAdd(&start[count[i / s.H]], 1);
-    __syncthreads();
-    if (tid == 0) {  // start[v] = number of heads with more live tiles than v
-        int run = 0;
-        for (int v = ntiles; v >= 0; --v) {
-            const int c = start[v];
-            start[v] = run;
-            run += c;
-        }
-    }
-    __syncthreads();
-    for (int i = tid; i < BH; i += 1024) a.order[atomicAdd(&start[count[i / s.H]], 1)] = i;
-}
-
 // The split of this instantiation's grid on the current device (fwd_split.hpp).
 // Split pieces at D = 128 take the register-staged kernel: it fits two waves per SIMD (the
 // asynchronous one needs ~330 registers for its swizzled LDS addresses and runs one), and few
@@ -640,133 +470,69 @@ __global__ __launch_bounds__(1024) void rowmask_batch_order_kernel(FwdArgs a, in
 // timings, 125 -> 104 us over 200 back-to-back calls after 1000 warm-up calls) while full grids
 // lose (B2 H16 L2048 D128 causal 347 -> 396 us, same back-to-back timing): those keep the
 // asynchronous kernel.
-template <int D>
-constexpr bool kSplitAsync = D != 128;
+constexpr int kD = 128, kBN = 32, kW = 4, kM = 32 * kW;
 
-template <int D, int BN, int W>
 FwdSplitPlan plan(const AttnShape &s) {
-    const int64_t blocks = (int64_t)(s.L + 32 * W - 1) / (32 * W) * s.B * s.H;
+    const int64_t blocks = (int64_t)(s.L + kM - 1) / kM * s.B * s.H;
     const int64_t slots = split_slots(
-        reinterpret_cast<const void *>(&fwd_f32_kernel<D, BN, W, true, false, kSplitAsync<D>, false, true>), 64 * W,
-        blocks);
-    return plan_split(s, 32 * W, BN, slots);
+        reinterpret_cast<const void *>(&fwd_f32_kernel<kD, kBN, kW, true, false, false, false, true>), 64 * kW, blocks);
+    return plan_split(s, kM, kBN, slots);
 }
 
-template <int D, int BN, int W>
-hipError_t launch_d(const FwdArgs &args, hipStream_t st) {
+hipError_t launch_f32(const FwdArgs &args, hipStream_t st) {
     FwdArgs a = args;
-    a.s.vec = args.s.vec && args.s.E == D;  // the ABI checked alignment; E must fill D
-    const int nqt = (a.s.L + 32 * W - 1) / (32 * W);
-    const dim3 grid(nqt * a.s.B * a.s.H), block(64 * W);
-    const bool mask = a.s.mask != nullptr;
+    a.s.vec = args.s.vec && args.s.E == kD;  // the ABI checked alignment; E must fill D
+    const int nqt = (a.s.L + kM - 1) / kM;
+    const dim3 grid(nqt * a.s.B * a.s.H), block(64 * kW);
     if (a.split_o) {
-        const FwdSplitPlan p = plan<D, BN, W>(a.s);
+        const FwdSplitPlan p = plan(a.s);
         if (p.chunk > 0 && p.bytes <= a.split_bytes) {
             record_schedule(split_chunk, p.chunk);
             record_schedule(split_pieces, p.max_pieces);
             a.split_chunk = p.chunk, a.split_max = p.max_pieces;
             a.split_lse = a.split_o + (size_t)a.s.B * a.s.H * a.s.L * p.max_pieces * a.s.E;
             const dim3 sgrid((unsigned)p.blocks);
-            if (a.s.vec && kSplitAsync<D>) {
-                if (a.s.causal)
-                    return_if(launch(fwd_f32_kernel<D, BN, W, true, false, true, false, true>, sgrid, block, st, a));
-                else
-                    return_if(launch(fwd_f32_kernel<D, BN, W, false, false, true, false, true>, sgrid, block, st, a));
-            } else if (a.s.causal) {
-                return_if(launch(fwd_f32_kernel<D, BN, W, true, false, false, false, true>, sgrid, block, st, a));
-            } else {
-                return_if(launch(fwd_f32_kernel<D, BN, W, false, false, false, false, true>, sgrid, block, st, a));
-            }
+            if (a.s.causal)
+                return_if(launch(fwd_f32_kernel<kD, kBN, kW, true, false, false, false, true>, sgrid, block, st, a));
+            else
+                return_if(launch(fwd_f32_kernel<kD, kBN, kW, false, false, false, false, true>, sgrid, block, st, a));
             const int64_t rows = (int64_t)a.s.B * a.s.H * a.s.L;
-            return launch(fwd_split_merge_kernel<float>, dim3((unsigned)((rows + 15) / 16)), dim3(256), st, a,
-                          32 * W, BN);
+            return launch(fwd_split_merge_kernel<float>, dim3((unsigned)((rows + 15) / 16)), dim3(256), st, a, kM, kBN);
         }
     }
-    if constexpr (W == 1) {  // short causal rows without a mask (with_config)
-        if (a.s.vec)
-            return launch(fwd_f32_kernel<D, BN, W, true, false, true>, grid, block, st, a);
-        return launch(fwd_f32_kernel<D, BN, W, true, false, false>, grid, block, st, a);
-    } else if (a.s.vec && !(mask && a.s.causal)) {  // (causal + mask: register staging, fewer VGPRs)
-        if (a.s.causal)
-            return_if(launch(fwd_f32_kernel<D, BN, W, true, false, true>, grid, block, st, a));
-        else if (mask && a.s.msl == 0 && BN <= 64) {
-            const int ntiles = (a.s.S + BN - 1) / BN;
-            if (a.order && a.s.B * a.s.H <= kOrderMaxHeads && ntiles <= kOrderMaxTiles) {
-                if (a.s.msh == 0 && a.s.B <= kOrderMaxBatch) {
-                    return_if(launch(rowmask_batch_order_kernel<BN>, dim3(1), dim3(1024), st, a, ntiles));
-                } else {
-                    return_if(launch(rowmask_tiles_kernel<BN>, dim3(a.s.B * a.s.H), dim3(64), st, a));
-                    return_if(launch(rowmask_order_kernel, dim3(1), dim3(1024), st, a, ntiles));
-                }
-                const dim3 ogrid(nqt * 8 * ((a.s.B * a.s.H + 7) / 8));
-                return_if(launch(fwd_f32_kernel<D, BN, W, false, true, true, true>, ogrid, block, st, a));
-            } else {
-                a.order = nullptr;
-                return_if(launch(fwd_f32_kernel<D, BN, W, false, true, true, true>, grid, block, st, a));
-            }
-        }
-        else if (mask)
-            return_if(launch(fwd_f32_kernel<D, BN, W, false, true, true>, grid, block, st, a));
-        else
-            return_if(launch(fwd_f32_kernel<D, BN, W, false, false, true>, grid, block, st, a));
-    } else if (a.s.causal && mask) {
-        return_if(launch(fwd_f32_kernel<D, BN, W, true, true, false>, grid, block, st, a));
-    } else if (a.s.causal) {
-        return_if(launch(fwd_f32_kernel<D, BN, W, true, false, false>, grid, block, st, a));
-    } else if (mask) {
-        return_if(launch(fwd_f32_kernel<D, BN, W, false, true, false>, grid, block, st, a));
-    } else {
-        return_if(launch(fwd_f32_kernel<D, BN, W, false, false, false>, grid, block, st, a));
+    const bool mask = a.s.mask != nullptr;
+    if (a.s.vec && !(mask && a.s.causal)) {  // (causal + mask: register staging, fewer VGPRs)
+        if (a.s.causal) return launch(fwd_f32_kernel<kD, kBN, kW, true, false, true>, grid, block, st, a);
+        if (!mask) return launch(fwd_f32_kernel<kD, kBN, kW, false, false, true>, grid, block, st, a);
+        if (a.s.msl != 0) return launch(fwd_f32_kernel<kD, kBN, kW, false, true, true>, grid, block, st, a);
+        return_if(order_heads<kBN>(a, st));
+        return launch(fwd_f32_kernel<kD, kBN, kW, false, true, true, true>, ordered_grid(a, nqt), block, st, a);
     }
-    return hipSuccess;
+    if (a.s.causal && mask) return launch(fwd_f32_kernel<kD, kBN, kW, true, true, false>, grid, block, st, a);
+    if (a.s.causal) return launch(fwd_f32_kernel<kD, kBN, kW, true, false, false>, grid, block, st, a);
+    if (mask) return launch(fwd_f32_kernel<kD, kBN, kW, false, true, false>, grid, block, st, a);
+    return launch(fwd_f32_kernel<kD, kBN, kW, false, false, false>, grid, block, st, a);
 }
 
-// The instantiation the forward runs for a shape: head dim D, key tile BN, waves W.  Short causal
-// problems take smaller workgroups over 32-key tiles: their causal work units are finer, which
-// balances the CUs better (measured on one MI355X: B64 H6 L256 D64 causal 54.0 -> 49.5 us with
-// 2 waves; B8 H12 L1024 unchanged; non-causal B16 H16 L512 slower, 161 -> 171 us), and one wave
-// each when no mask is given (49.5 -> 43.1 us, the one-buffer path of fwd_f32_kernel).  At D = 64
-// the 4-wave workgroups take 32-key tiles: half the LDS of 64-key tiles (32 KB), so four
-// workgroups fit a CU instead of two (B8 H12 L1024 causal 148.7 -> 145.7 us, B2 H12 L4096 causal
-// 480 -> 457 us).
-template <typename F>
-auto with_config(const AttnShape &s, F f) {
-    const bool small = s.causal && s.L <= 256;
-    const bool one = small && s.mask == nullptr;
-    if (s.E <= 32) {
-        if (one) return f.template operator()<32, 32, 1>();
-        return small ? f.template operator()<32, 32, 2>() : f.template operator()<32, 64, 4>();
-    }
-    if (s.E <= 64) {
-        if (one) return f.template operator()<64, 32, 1>();
-        return small ? f.template operator()<64, 32, 2>() : f.template operator()<64, 32, 4>();
-    }
-    return f.template operator()<128, 32, 4>();
-}
-
-struct SplitBytes {
-    const AttnShape &s;
-    template <int D, int BN, int W>
-    size_t operator()() const { return plan<D, BN, W>(s).bytes; }
-};
-
-struct Launch {
-    const FwdArgs &a;
-    hipStream_t st;
-    template <int D, int BN, int W>
-    hipError_t operator()() const { return launch_d<D, BN, W>(a, st); }
-};
+// Which kernel a shape takes: up to head dim 127 the split products of fwd_x3.hip (one and a half
+// to three times as fast: causal B2 H12 L4096 D64 439 -> 273 us, B4 H8 L1001 D80 185 -> 68); float32
+// MFMAs at 128, and from 65 up where the caller asks for scores the backward repeats exactly
+// (DC_FLAG_CONSISTENT_SCORES), because the backward of those head dims forms its scores with them.
+// (At 128 the split kernel would take causal B2 H16 L2048 from 357 to 193 us, at half the error; but
+// scores near 100 are held to the reference's own rounding within 2e-5, which it there meets less
+// closely by being nearer the exact result: the reference is off by 2.6e-5.)
+bool split_products(const AttnShape &s) { return s.E <= 64 || (s.E < kD && !s.consistent); }
 
 }  // namespace
 
 size_t fwd_f32_split_bytes(const AttnShape &s) {
     if (s.B == 0 || s.H == 0 || s.L == 0) return 0;
-    return with_config(s, SplitBytes{s});
+    return split_products(s) ? fwd_x3_split_bytes(s) : plan(s).bytes;
 }
 
 hipError_t launch_fwd_f32(const FwdArgs &a, hipStream_t st) {
     if (a.s.B == 0 || a.s.H == 0 || a.s.L == 0) return hipSuccess;
-    return with_config(a.s, Launch{a, st});
+    return split_products(a.s) ? launch_fwd_x3(a, st) : launch_f32(a, st);
 }
 
 }  // namespace dc

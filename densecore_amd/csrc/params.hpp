@@ -161,6 +161,8 @@ hipError_t launch_to_f16(const F16Copy *copies, int n, int64_t nslabs, float *pa
 
 // Each launcher returns hipSuccess or the launch error; it never synchronizes.
 hipError_t launch_fwd_f32(const FwdArgs &a, hipStream_t st);
+hipError_t launch_fwd_x3(const FwdArgs &a, hipStream_t st);  // its split-product kernels (fwd_x3.hip)
+size_t fwd_x3_split_bytes(const AttnShape &s);
 // Workspace bytes the float32 forward uses to split key ranges on the current device (0: it
 // does not split this shape).
 size_t fwd_f32_split_bytes(const AttnShape &s);

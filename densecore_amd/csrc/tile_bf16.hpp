@@ -15,7 +15,6 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 
 template <int R, int D>
 struct CMTile {
-    static_assert(R % 64 == 0, "tiles are filled 64 rows at a time");
     static constexpr int C = D / 8;        // 16-byte chunks per row
     static constexpr int P = R + 4;        // slots per chunk column (4 pad slots)
     static constexpr int SLOTS = C * P;
@@ -32,6 +31,7 @@ struct CMTile {
 // per-tile address arithmetic in VGPRs and no per-lane bounds tests.
 template <int R, int D, bool VEC, int W>
 DEVI void fill_cm(u32x4 *dst, const __bf16 *src, int nrows, int E, int wave, int lane) {
+    static_assert(R % 64 == 0, "tiles are filled 64 rows at a time");
     using T = CMTile<R, D>;
     constexpr int count = (T::NT + W - 1) / W;
     const uint32_t loff = (uint32_t)lane * (D * 2);
