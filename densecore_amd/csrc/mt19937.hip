@@ -28,6 +28,8 @@
 // The jump polynomials (128 of them) are computed once on the host: phi by Berlekamp-Massey on
 // 2 * 19937 bits of the stream, then z^(digit * 2^(17 + 6 level)) mod phi by squaring and
 // multiplying; the caller uploads them into its own device buffer (dc_mt19937_table_init).
+#include <climits>
+#include <type_traits>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -214,15 +216,6 @@ DEVI bool keep(uint32_t hi, uint32_t lo, uint64_t thr) {
     return r < thr;
 }
 
-// Orders this wave's LDS accesses around it (the LDS executes one wave's instructions in order,
-// so the compiler is the only thing that could move a read above another lane's write): the
-// wave-scope release / wave barrier / acquire sequence, no wait on global stores.
-DEVI void wave_lds_order() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // One workgroup: the current block `state` (positions 0..623), the words after it up to
 // A0 + 623, the head's keep bits, the window at A0, and (when the last drawn output lies before
 // A0) the engine block that holds it.
@@ -257,73 +250,101 @@ __global__ __launch_bounds__(256) void mt_base_kernel(MtArgs a) {
         for (int i = tid; i < kState; i += 256) a.state[i] = x[a.state_block * kState + i];
 }
 
-// One workgroup per destination window: dst[w] = W(src[w / 64] + digit * step), digit = w % 64,
-// with g = table[level][digit].  The sequence seq[i] = x[src + i], i < 20576, is generated into
-// LDS once; wave v sums the g-terms of i in its eighth of [0, 19937): lanes < 52 own 12
-// consecutive output words each and read a 20-word window of seq per group of 8 terms; the
-// eight partial windows are then XORed together.
-constexpr int kSeqWords = 20576;                        // >= 19937 + 624 + 15, a multiple of 8
+// dst window w = W(src window w / 64 + digit * step), digit = w % 64, with g = table[level][digit],
+// by `split` workgroups: each generates the sequence seq[i] = x[src + i] into LDS as far as it needs
+// it and its eight waves sum g's terms over a 1/(8 split) part of [0, 19937); lanes < 52 own 12
+// consecutive output words each and read a 20-word window of seq per group of 8 terms.  The eight
+// partial windows are XORed, and the workgroups' ones stand side by side in dst (`src_split` of
+// them in src), XORed by whoever reads them.
+// Bound: VALU (about 6 M XORs per jump) and, in a launch of few jumps, one workgroup's latency, so
+// the level-1 jumps (at most 64) are split over 8 workgroups each: 98 -> 1L us for the 6 of 25 M
+// draws.  The sequence is 20576 words, 96 more than half of a CU's LDS: its last words are made
+// after the terms that read the first ones are summed, in their place, and two workgroups share a
+// CU.  Both launches for 25 M draws (6 level-1, 384 level-0 jumps): 300 -> 143 us.
+constexpr int kSeqWords = 20480;  // LDS: half a CU's
+constexpr int kTailWords = 96;    // words past it that the last terms read (kDegree - 1 + 12 * 51 + 19)
 constexpr int kJumpWaves = 8;
-constexpr int kGroups = (kDegree + 7) / 8;              // groups of 8 terms
-constexpr int kGroupsPerWave = (kGroups + kJumpWaves - 1) / kJumpWaves;
 constexpr int kOwn = 12, kOwners = kState / kOwn;       // 52 owner lanes per wave
+constexpr int kTailTerms = 620 * 32;                    // terms from here on read past kSeqWords
+static_assert(kTailTerms - 1 + kOwn * (kOwners - 1) + kOwn + 8 < kSeqWords, "terms before the tail stay inside");
+static_assert(kDegree - 1 + kOwn * (kOwners - 1) + kOwn + 8 < kSeqWords + kTailWords && kTailWords <= 227, "one step makes the tail");
 
-__global__ __launch_bounds__(512) void mt_jump_kernel(const uint32_t *src, uint32_t *dst,
-                                                      const uint32_t *table, int level, int count) {
+__global__ __launch_bounds__(512) void mt_jump_kernel(const uint32_t *src, int src_split, uint32_t *dst,
+                                                      const uint32_t *table, int level, int count, int split) {
     __shared__ __align__(16) uint32_t seq[kSeqWords];
-    const int w = blockIdx.x;
+    const int w = blockIdx.x / split, part = blockIdx.x % split;
     if (w >= count) return;
     const int digit = w % kRadix;
-    const uint32_t *in = src + (size_t)(w / kRadix) * kState;
-    uint32_t *out = dst + (size_t)w * kState;
+    const uint32_t *in = src + (size_t)(w / kRadix) * src_split * kState;
+    uint32_t *out = dst + ((size_t)w * split + part) * kState;
     const int tid = threadIdx.x;
+    auto first = [&](int i) {
+        uint32_t x = 0;
+        for (int k = 0; k < src_split; ++k) x ^= in[(size_t)k * kState + i];
+        return x;
+    };
     if (digit == 0) {
-        for (int i = tid; i < kState; i += 512) out[i] = in[i];
+        for (int i = tid; i < kState; i += 512) out[i] = part == 0 ? first(i) : 0u;
         return;
     }
     const uint32_t *g = table + ((size_t)level * kRadix + digit) * kTableWords;
-    for (int i = tid; i < kState; i += 512) seq[i] = in[i];
+    // Words of g (32 terms each) per wave; this wave's are [w0, w1).
+    const int per_wave = (kTableWords + kJumpWaves * split - 1) / (kJumpWaves * split);
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int w0 = min(kTableWords, (part * kJumpWaves + wave) * per_wave), w1 = min(kTableWords, w0 + per_wave);
+    const int block_end = min(kTableWords, (part + 1) * kJumpWaves * per_wave);
+    const int need = min(kSeqWords, 32 * block_end + kState + 16);
+    for (int i = tid; i < kState; i += 512) seq[i] = first(i);
     __syncthreads();
-    for (int base = kState; base < kSeqWords; base += 227) {  // x[u] needs x[u - 227]: 227 at a time
+    for (int base = kState; base < need; base += 227) {  // x[u] needs x[u - 227]: 227 at a time
         const int u = base + tid;
         if (tid < 227 && u < kSeqWords) seq[u] = seq[u - 227] ^ twist_d(seq[u - 624], seq[u - 623]);
         __syncthreads();
     }
     // Every lane runs the sum (lanes past the owners repeat the last owner's words and store
     // nothing), so the group index and the polynomial bits are wave-uniform: the bits come from
-    // two VGPRs loaded up front (word w of this wave's 78 at lane w % 64 of gw[w / 64]) through
+    // two VGPRs loaded up front (word w of this wave's at lane w % 64 of gw[w / 64]) through
     // readlane, and the term tests are scalar branches.
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int j0 = kOwn * (lane < kOwners ? lane : kOwners - 1);
-    const int g_begin = wave * kGroupsPerWave;
-    const int g_end = g_begin + kGroupsPerWave < kGroups ? g_begin + kGroupsPerWave : kGroups;
-    static_assert(kGroupsPerWave % 4 == 0 && kGroupsPerWave / 4 <= 128, "g words per wave");
-    const int w0 = g_begin / 4;  // first g word of this wave (4 groups of 8 bits per word)
-    const uint32_t gw0 = w0 + lane < kTableWords ? g[w0 + lane] : 0u;
-    const uint32_t gw1 = w0 + 64 + lane < kTableWords ? g[w0 + 64 + lane] : 0u;
+    const uint32_t gw0 = w0 + lane < w1 ? g[w0 + lane] : 0u;
+    const uint32_t gw1 = w0 + 64 + lane < w1 ? g[w0 + 64 + lane] : 0u;
     uint32_t acc[kOwn];
 #pragma unroll
     for (int u = 0; u < kOwn; ++u) acc[u] = 0;
-    for (int gi = g_begin; gi < g_end; ++gi) {
-        const int wi = (gi >> 2) - w0;
-        const uint32_t word = wi < 64 ? __builtin_amdgcn_readlane(gw0, wi)
-                                      : __builtin_amdgcn_readlane(gw1, wi - 64);
-        const uint32_t gb = (word >> (8 * (gi & 3))) & 0xffu;  // g bits 8 gi .. 8 gi + 7
-        if (gb == 0) continue;
-        uint32_t win[kOwn + 8];  // seq[8 gi + j0 + 0 .. 19]: five 16-byte reads
+    auto terms = [&](int wi, bool wrap) {  // word w0 + wi of g
+        const uint32_t word = wi < 64 ? __builtin_amdgcn_readlane(gw0, wi) : __builtin_amdgcn_readlane(gw1, wi - 64);
 #pragma unroll
-        for (int u = 0; u < kOwn + 8; u += 4) {
-            const u32x4 x = *reinterpret_cast<const u32x4 *>(&seq[8 * gi + j0 + u]);
-            win[u] = x[0], win[u + 1] = x[1], win[u + 2] = x[2], win[u + 3] = x[3];
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t gb = (word >> (8 * k)) & 0xffu;
+            if (gb == 0) continue;
+            const int base = 32 * (w0 + wi) + 8 * k + j0;
+            uint32_t win[kOwn + 8];  // seq[base + 0 .. 19]: five 16-byte reads
+#pragma unroll
+            for (int u = 0; u < kOwn + 8; u += 4) {
+                const int at = base + u - (wrap && base + u >= kSeqWords ? kSeqWords : 0);
+                const u32x4 x = *reinterpret_cast<const u32x4 *>(&seq[at]);
+                win[u] = x[0], win[u + 1] = x[1], win[u + 2] = x[2], win[u + 3] = x[3];
+            }
+#pragma unroll
+            for (int d = 0; d < 8; ++d)
+                if (gb >> d & 1u)
+#pragma unroll
+                    for (int u = 0; u < kOwn; ++u) acc[u] ^= win[d + u];
         }
-#pragma unroll
-        for (int d = 0; d < 8; ++d)
-            if (gb >> d & 1u)
-#pragma unroll
-                for (int u = 0; u < kOwn; ++u) acc[u] ^= win[d + u];
+    };
+    constexpr int kTailWord = kTailTerms / 32;
+    for (int wi = 0; wi < min(w1, kTailWord) - w0; ++wi) terms(wi, false);
+    __syncthreads();  // every wave is done with the sequence's start
+    if (block_end > kTailWord) {
+        if (tid < kTailWords) {
+            const int u = kSeqWords + tid;
+            seq[tid] = seq[u - 227] ^ twist_d(seq[u - 624], seq[u - 623]);
+        }
+        __syncthreads();
+        for (int wi = max(0, kTailWord - w0); wi < w1 - w0; ++wi) terms(wi, true);
+        __syncthreads();
     }
-    __syncthreads();  // every wave is done with seq: reuse it for the partial windows
-    if (lane < kOwners)
+    if (lane < kOwners)  // seq is free: the waves' partial windows
 #pragma unroll
         for (int u = 0; u < kOwn; ++u) seq[wave * kState + j0 + u] = acc[u];
     __syncthreads();
@@ -335,125 +356,88 @@ __global__ __launch_bounds__(512) void mt_jump_kernel(const uint32_t *src, uint3
     }
 }
 
-// One wave per pair of chunks, one chunk per half-wave (chunks 2 b and 2 b + 1): each half
-// makes 64 words (32 elements, one word of keep bits) per step from its chunk's window in its own
-// LDS ring.  A word depends on the word 227 before it, so a step's words depend only on steps
-// three or more back: one LDS ordering point every three steps is enough, and the three steps
-// between them overlap their LDS latency.
-struct Half {
-    int64_t e_begin;  // first element of the chunk
-    int n;            // elements of the chunk
-    int words;        // words to make: 2 n, or up to the end of the engine block it writes back
-    int sb;           // that block's first word (relative), or -1
-};
+// One workgroup per chunk, which makes kStep words (96 elements, three words of keep bits) per step
+// from its window, in an LDS ring: a word depends on the word 227 before it, so a step's words
+// depend only on earlier steps'.  Bound by the latency of a step (LDS read, twist, LDS write,
+// barrier), so two waves do nothing else, and two more temper and test the words of the step
+// before.  (Two chunks per wave, three times 32 elements between LDS ordering points: 371 us for 25 M
+// draws, at an eighth of the waves the device holds; two waves that do both: 204 us; now 128 us.)
+constexpr int kStep = 192;
 
-DEVI Half half_of(const MtArgs &a, int c, int chunks) {
-    Half h{0, 0, 0, -1};
-    if (c >= chunks) return h;
-    h.e_begin = a.eh + (int64_t)c * (kChunkWords / 2);
-    const int64_t n = a.n - h.e_begin;
-    h.n = n < kChunkWords / 2 ? (int)n : kChunkWords / 2;
-    h.words = 2 * h.n;
+__global__ __launch_bounds__(256) void mt_chunk_kernel(MtArgs a, const uint32_t *wins) {
+    __shared__ __align__(16) uint32_t ring[1024];
+    const int tid = threadIdx.x & 127, lane = tid & 63;  // of the generating, or the testing, pair of waves
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool generate = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7) == 0;
+    const int c = blockIdx.x;
+    const int64_t e_begin = a.eh + (int64_t)c * (kChunkWords / 2);  // first element, a multiple of 64
+    const int n = (int)min(a.n - e_begin, (int64_t)(kChunkWords / 2));
+    int words = 2 * n;  // words to make: all elements', or up to the end of the engine block it writes back
+    int sb = -1;        // that block's first word
     const int64_t chunk_pos = a.a0 + (int64_t)c * kChunkWords;  // relative position of word 0
     if (a.state_block >= 0 && a.state_block * (int64_t)kState >= a.a0) {
-        const int64_t sb = a.state_block * (int64_t)kState - chunk_pos;
-        if (sb >= 0 && sb < kChunkWords) {
-            h.sb = (int)sb;
-            if (h.sb + kState > h.words) h.words = h.sb + kState;
+        const int64_t at = a.state_block * (int64_t)kState - chunk_pos;
+        if (at >= 0 && at < kChunkWords) {
+            sb = (int)at;
+            words = max(words, sb + kState);
         }
     }
-    return h;
-}
-
-__global__ __launch_bounds__(64) void mt_chunk_kernel(MtArgs a, const uint32_t *wins, int chunks) {
-    __shared__ __align__(16) uint32_t rings[2][1024];
-    const int lane = threadIdx.x, half = lane >> 5, hl = lane & 31;
-    const int c = 2 * blockIdx.x + half;
-    const Half hh = half_of(a, c, chunks);
-    const int words_max = max(half_of(a, 2 * blockIdx.x, chunks).words,
-                              half_of(a, 2 * blockIdx.x + 1, chunks).words);
-    uint32_t *ring = rings[half];
-    if (c < chunks) {
-        const uint32_t *win = wins + (size_t)c * kState;
-        for (int i = hl; i < kState; i += 32) ring[i] = win[i];
-    }
-    wave_lds_order();
-    uint32_t *bits = a.bits + (hh.e_begin >> 5);  // e_begin is a multiple of 64
+    for (int i = threadIdx.x; i < kState; i += 256) ring[i] = wins[(size_t)c * kState + i];
+    __syncthreads();
+    uint32_t *bits = a.bits + (e_begin >> 5);
     const uint64_t thr = a.thr;
-    // Keep bits of the pair (w0, w1) at words u0, u0 + 1 of this half's step starting at base.
-    auto emit = [&](int base, uint32_t w0, uint32_t w1) {
-        const int e = base / 2 + hl;
-        const uint64_t r = (((uint64_t)temper(w0) << 32) | temper(w1)) & ((1ull << 53) - 1);
-        const uint64_t m = __ballot(e < hh.n && r < thr);
-        if (hl == 0 && base / 2 < hh.n) bits[base / 64] = (uint32_t)(m >> (32 * half));
-    };
-    auto make = [&](int u0, uint32_t &w0, uint32_t &w1) {
-        const uint32_t x0 = ring[(u0 - 624) & 1023], x1 = ring[(u0 - 623) & 1023];
-        const uint32_t x2 = ring[(u0 - 622) & 1023];
-        w0 = ring[(u0 - 227) & 1023] ^ twist_d(x0, x1);
-        w1 = ring[(u0 - 226) & 1023] ^ twist_d(x1, x2);
-        *reinterpret_cast<uint2 *>(&ring[u0 & 1023]) = make_uint2(w0, w1);
-    };
-    // Words 0 .. 639: the window, then the first generated words (which read only the window).
-    for (int base = 0; base < 640; base += 64) {
-        const int u0 = base + 2 * hl;
-        uint32_t w0, w1;
-        if (u0 < kState) {
-            w0 = ring[u0];
-            w1 = ring[u0 + 1];
-        } else {
-            make(u0, w0, w1);
+    const int pair = min(tid, kStep / 2 - 1);  // this lane's element of a step (the last 32 lanes repeat one)
+    // Steps start at words 0, 192, 384 (the window's), 576 (its last 48 and the first made from it),
+    // 768, ..., `last`.
+    const int last = words <= 576 + kStep ? 576 : 576 + (words - 577) / kStep * kStep;
+    if (generate) {
+        const int u0 = 576 + 2 * pair;
+        // The last 32 lanes write their element's words again: the same values.
+        auto make = [&](int u) {
+            const uint32_t x0 = ring[(u - 624) & 1023], x1 = ring[(u - 623) & 1023], x2 = ring[(u - 622) & 1023];
+            const uint32_t y0 = ring[(u - 227) & 1023], y1 = ring[(u - 226) & 1023];
+            *reinterpret_cast<uint2 *>(&ring[u & 1023]) = make_uint2(y0 ^ twist_d(x0, x1), y1 ^ twist_d(x1, x2));
+        };
+        if (u0 >= kState) make(u0);
+        __syncthreads();
+        for (int u = u0 + kStep; u <= last + 2 * pair; u += kStep) {
+            make(u);
+            __syncthreads();
         }
-        emit(base, w0, w1);
+        return;
     }
-    wave_lds_order();
-    bool captured = false;
-    for (int base = 640; base < words_max; base += 192) {
-        // All reads of the three steps first (none of them reads a word the three steps
-        // write), then the words, the ring writes and the keep bits.
-        uint32_t x[3][5];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int u0 = base + 64 * k + 2 * hl;
-            x[k][0] = ring[(u0 - 624) & 1023];
-            x[k][1] = ring[(u0 - 623) & 1023];
-            x[k][2] = ring[(u0 - 622) & 1023];
-            x[k][3] = ring[(u0 - 227) & 1023];
-            x[k][4] = ring[(u0 - 226) & 1023];
+    // Keep bits of the step at `base`: wave 0 holds 64 elements, wave 1 the other 32; lanes 0 and 1 (lane
+    // 0 of wave 1) store a word each.  FULL: every element of the step is the chunk's.
+    auto emit = [&](int base, auto full) {
+        constexpr bool FULL = decltype(full)::value;
+        const uint2 x = *reinterpret_cast<const uint2 *>(&ring[(base + 2 * pair) & 1023]);
+        const uint64_t r = (((uint64_t)temper(x.x) << 32) | temper(x.y)) & ((1ull << 53) - 1);
+        const bool valid = FULL | (base / 2 + tid < n);
+        const uint64_t m = __ballot(valid & (r < thr));
+        const int word = base / 64 + 2 * wave + lane;
+        if (lane < 2 - wave && (FULL || 32 * word < n)) bits[word] = (uint32_t)(m >> (32 * lane));
+    };
+    const std::true_type whole;
+    const std::false_type cut;
+    // The step after which the ring holds the whole engine block this chunk writes back (it is copied
+    // then: at most 624 + 191 words were made since its first, and the next step's take older places).
+    const int block_at = sb < 0 ? INT_MAX : max(576, 576 + (sb + kState - kStep - 576 + kStep - 1) / kStep * kStep);
+    const int full_end = n >= kStep / 2 ? 2 * n - kStep : -1;  // the last base whose elements are all the chunk's
+    for (int base = 0; base < 576; base += kStep) emit(base, cut);
+    __syncthreads();
+    int base = 576;  // made: its step, while the next one's is being made
+    for (;;) {
+        for (; base < min(last, block_at) && base <= full_end; base += kStep) {
+            emit(base, whole);
+            __syncthreads();
         }
-        // Three independent chains, straight-line: words, ring writes, keep ballots; then the
-        // (branching) stores of the three keep words.
-        uint32_t w[3][2];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            w[k][0] = x[k][3] ^ twist_d(x[k][0], x[k][1]);
-            w[k][1] = x[k][4] ^ twist_d(x[k][1], x[k][2]);
-        }
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            *reinterpret_cast<uint2 *>(&ring[(base + 64 * k + 2 * hl) & 1023]) = make_uint2(w[k][0], w[k][1]);
-        uint64_t m[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const int e = (base + 64 * k) / 2 + hl;
-            const uint64_t r = (((uint64_t)temper(w[k][0]) << 32) | temper(w[k][1])) & ((1ull << 53) - 1);
-            m[k] = __ballot(e < hh.n && r < thr);
-        }
-        if (hl == 0) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-                if ((base + 64 * k) / 2 < hh.n) bits[(base + 64 * k) / 64] = (uint32_t)(m[k] >> (32 * half));
-        }
-        wave_lds_order();
-        // The engine block this chunk writes back: copied once its last word is made (the ring
-        // still holds it: at most 624 + 191 words were made since its first).
-        if (hh.sb >= 0 && !captured && base + 192 >= hh.sb + kState) {
-            for (int i = hl; i < kState; i += 32) a.state[i] = ring[(hh.sb + i) & 1023];
-            captured = true;
-        }
+        if (base == block_at)
+            for (int i = tid; i < kState; i += 128) a.state[i] = ring[(sb + i) & 1023];
+        emit(base, cut);
+        if (base >= last) break;
+        __syncthreads();
+        base += kStep;
     }
-    if (hh.sb >= 0 && !captured)  // the block lies within words 0 .. 639
-        for (int i = hl; i < kState; i += 32) a.state[i] = ring[(hh.sb + i) & 1023];
 }
 
 // y = x * (keep ? scale : 0): the reference's input * noise, noise = bernoulli / float32(1 - p)
@@ -480,10 +464,13 @@ __global__ __launch_bounds__(256) void dropout_apply4_kernel(const uint32_t *bit
 
 }  // namespace
 
+// Workgroups per level-1 jump.
+constexpr int kLevel1Split = 8;
+
 size_t window_words(int chunks) {
     if (chunks == 0) return kState;
     const int n1 = (chunks + kRadix - 1) / kRadix;
-    return (size_t)(1 + n1 + chunks) * kState;
+    return (size_t)(1 + n1 * kLevel1Split + chunks) * kState;
 }
 
 bool tables_ready() { return tables().ok; }
@@ -509,12 +496,13 @@ hipError_t launch_bernoulli(const MtArgs &a, const uint32_t *table, int chunks, 
     return_if(launch(mt_base_kernel, dim3(1), dim3(256), st, a));
     if (chunks == 0) return hipSuccess;
     // Radix-64 tree: level 1 (c1), then level 0 (c0).  Window arrays are carved from `wins`
-    // (window_words(chunks) words): [W(A0)] [n1 level-1 windows] [chunk windows].
+    // (window_words(chunks) words): [W(A0)] [n1 level-1 windows, in parts] [chunk windows].
     const int n1 = (chunks + kRadix - 1) / kRadix;
-    uint32_t *l1 = wins + kState, *l0 = l1 + (size_t)n1 * kState;
-    return_if(launch(mt_jump_kernel, dim3(n1), dim3(512), st, (const uint32_t *)wins, l1, table, 1, n1));
-    return_if(launch(mt_jump_kernel, dim3(chunks), dim3(512), st, (const uint32_t *)l1, l0, table, 0, chunks));
-    return launch(mt_chunk_kernel, dim3((chunks + 1) / 2), dim3(64), st, a, (const uint32_t *)l0, chunks);
+    uint32_t *l1 = wins + kState, *l0 = l1 + (size_t)n1 * kLevel1Split * kState;
+    return_if(launch(mt_jump_kernel, dim3(n1 * kLevel1Split), dim3(512), st, (const uint32_t *)wins, 1, l1, table, 1, n1,
+                     kLevel1Split));
+    return_if(launch(mt_jump_kernel, dim3(chunks), dim3(512), st, (const uint32_t *)l1, kLevel1Split, l0, table, 0, chunks, 1));
+    return launch(mt_chunk_kernel, dim3(chunks), dim3(256), st, a, (const uint32_t *)l0);
 }
 
 hipError_t launch_dropout_apply(const uint32_t *bits, int64_t n, float scale, const float *x, float *y,
