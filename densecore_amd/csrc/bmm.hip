@@ -1,4 +1,4 @@
-// Float32 batched matrix product on CDNA4 MFMA (v_mfma_f32_32x32x2_f32): C[b] = A[b] B[b].
+// Float32 batched matrix product, C[b] = A[b] B[b], on the bf16 matrix cores (split products, x3.hpp).
 //
 // The reference registers one bmm kernel, (Cpu, Float32) (src/batched_matmul.rs:28-49), which runs
 // PyTorch's bmm on the operands' strided storage (src/torch_blas.rs:404-449): A is (batch, m, k),
@@ -7,106 +7,116 @@
 // math attention path's two products (q k^T, a transposed view of k, and weights v) and MHA's.
 //
 // Blocking (this kernel's own): a workgroup of 4 waves computes a BM x BN tile of one batch item
-// (waves 2 x 2, each (BM/2) x (BN/2) as 32 x 32 MFMA tiles), over k in steps of BK.  A and B
-// tiles are staged in LDS k-major ([k][m], [k][n]), so an MFMA operand is 32 consecutive floats
-// per half-wave (lane l takes A[m = l % 32][k = l / 32] and B[k = l / 32][n = l % 32]).  Global
-// loads follow the operand's contiguous dimension: 16-byte loads along m or n are stored as they
-// are; 16-byte loads along k are stored transposed (lanes along m or n, conflict-free); other
-// layouts load one element per lane.  The next k tile is loaded into registers while the current
-// one is multiplied (one barrier per k tile).  Where every tile has the same k extent (no causal
-// trimming of k) BK = 16: half the LDS of BK = 32, so four workgroups run per CU and four waves per
-// SIMD hide the loads' latency (on one MI355X, 32 items of 2048 x 256 x 2048: 705 -> 598 us; 256
-// items of 512 x 64 x 512: 148 -> 134 us).  Products whose tiles stop k at the diagonal (causal
-// modes 2 and 3) keep BK = 32 and two workgroups per CU: their longest tiles set the time, and
-// sharing a SIMD four ways slowed them (D = 256 causal P V 529 -> 610 us).  Accumulation is
-// float32 (the reference sums the products in k order; here the MFMA's order, within the float32
-// tolerance).  The launcher also serves the attention path of head dims above 128 (wide.hip),
-// which writes C through strides and can add A B into C.
+// (waves 2 x 2, each (BM/2) x (BN/2) as 32 x 32 MFMA tiles), over k in steps of 16, one MFMA's depth.
+// A thread loads 8 elements of each operand along its contiguous dimension, splits them and writes
+// them to LDS in chunks along that dimension (two buffers, one barrier per step, the next step's
+// loads in flight): chunks along k are read as they are, chunks along m or n transposed
+// (ds_read_b64_tr_b16), both giving a lane the same eight k.  Six MFMAs per 32 x 32 tile and step,
+// smallest products first.  Bound: the MFMAs (24 per wave and step at 128 x 128) beside the splits
+// (44 VALU instructions per operand and step); few k steps also by writing C.  On one MI355X, float32
+// MFMAs before -> now: 32 items of 2048 x 256 x 2048 588 -> 444 us (155 TFLOP/s), of 2048 x 2048 x
+// 256 606 -> 478, 4096^3 1139 -> 826; 256 items of 512 x 64 x 512 121 -> 104, of 512 x 512 x 64 125 ->
+// 112 (268 MB of C).  Relative error against float64: depth 64 1.45e-7 -> 1.10e-7, 4096 1.15e-6 ->
+// 1.00e-6 (the reference sums the products in k order).  The launcher also serves the attention path
+// of head dims above 128 (wide.hip), which writes C through strides and can add A B into C.
 #include "common.hpp"
 #include "params.hpp"
+#include "x3.hpp"
 
 namespace dc {
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kPad = 4;  // LDS row padding (floats): keeps 16-byte stores aligned
+constexpr int BK = 16;  // one MFMA's depth
 
-template <int BM, int BN, int BK>
-struct alignas(16) BmmSmem {
-    float a[2][BK][BM + kPad];
-    float b[2][BK][BN + kPad];
-};
-
-// How an operand's tile is loaded: CONTIG_K: 16-byte loads along k (stored transposed);
-// CONTIG_MN: 16-byte loads along m (A) or n (B); SCALAR: one element per lane, any strides.
+// How an operand's tile is loaded: CONTIG_K: 16-byte loads along k; CONTIG_MN: 16-byte loads along
+// m (A) or n (B); SCALAR: one element at a time, any strides.
 enum Layout { CONTIG_K = 0, CONTIG_MN = 1, SCALAR = 2 };
 
-// The register stage of one operand tile: R rows (m or n) by BK, from `p` (the batch item's base)
-// with strides (s_r along the rows, s_k along k); rows past `rows` and k past `kk` read zero.
-template <int R, int L, int BK>
-struct Stage {
-    static constexpr int N = R * BK / (L == SCALAR ? 1 : 4) / kThreads;
-    static_assert(N >= 1, "tile too small for the workgroup");
-    f32x4 v[L == SCALAR ? 1 : N];
-    float s[L == SCALAR ? N : 1];
+// One operand's tile: R rows (m or n) by BK, as three chunk-major bf16 planes (x3.hpp), its chunks
+// of 8 along the dimension it is loaded along.
+template <int R, int L>
+struct Operand {
+    static constexpr bool ALONG_K = L != CONTIG_MN;
+    typedef X3Tile<ALONG_K ? R : BK, ALONG_K ? BK : R> Tile;
+    typedef CMTile<ALONG_K ? R : BK, ALONG_K ? BK : R> Shape;
+    static constexpr int CHUNKS = R * BK / 8;  // at most one per thread
+    static_assert(CHUNKS <= kThreads, "a thread stages one chunk");
+    f32x4 x[2];
 
+    // This thread's chunk (row or k index r of the tile, chunk c), and whether it has one.
+    DEVI static bool place(int tid, int &r, int &c) {
+        const int grp = tid >> 3;  // two chunks of four rows per eight threads (X3Stage)
+        c = (tid & 1) + 2 * (grp % (Shape::C / 2));
+        r = ((tid >> 1) & 3) + 4 * (grp / (Shape::C / 2));
+        return CHUNKS == kThreads || tid < CHUNKS;
+    }
+    // From `p` (the batch item's base) with strides (s_r along the rows, s_k along k); rows past
+    // `rows` and k past `kk` read zero.
     DEVI void load(const float *p, int64_t s_r, int64_t s_k, int r0, int rows, int k0, int kk, int tid) {
-        if constexpr (L == CONTIG_K) {
+        int r, c;
+        if (!place(tid, r, c)) return;
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, r = i % R, c = (i / R) * 4;  // lanes along rows
-                const int rr = r0 + r, k = k0 + c;
-                v[j] = (rr < rows && k < kk) ? *reinterpret_cast<const f32x4 *>(p + rr * s_r + k)
-                                             : f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        } else if constexpr (L == CONTIG_MN) {
+        for (int h = 0; h < 2; ++h) {
+            x[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if constexpr (L == CONTIG_K) {
+                const int k = k0 + 8 * c + 4 * h;
+                if (r0 + r < rows && k < kk) x[h] = *reinterpret_cast<const f32x4 *>(p + (r0 + r) * s_r + k);
+            } else if constexpr (L == CONTIG_MN) {
+                const int rr = r0 + 8 * c + 4 * h;
+                if (rr < rows && k0 + r < kk) x[h] = *reinterpret_cast<const f32x4 *>(p + (k0 + r) * s_k + rr);
+            } else {
 #pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, c = (i % (R / 4)) * 4, k = i / (R / 4);
-                const int rr = r0 + c, kg = k0 + k;
-                v[j] = (rr < rows && kg < kk) ? *reinterpret_cast<const f32x4 *>(p + kg * s_k + rr)
-                                              : f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, r = i % R, k = i / R;
-                const int rr = r0 + r, kg = k0 + k;
-                s[j] = (rr < rows && kg < kk) ? p[rr * s_r + kg * s_k] : 0.f;
+                for (int e = 0; e < 4; ++e) {
+                    const int k = k0 + 8 * c + 4 * h + e;
+                    if (r0 + r < rows && k < kk) x[h][e] = p[(r0 + r) * s_r + k * s_k];
+                }
             }
         }
     }
-    DEVI void store(float (*t)[R + kPad], int tid) const {
-        if constexpr (L == CONTIG_K) {
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, r = i % R, c = (i / R) * 4;
-#pragma unroll
-                for (int u = 0; u < 4; ++u) t[c + u][r] = v[j][u];
-            }
-        } else if constexpr (L == CONTIG_MN) {
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, c = (i % (R / 4)) * 4, k = i / (R / 4);
-                *reinterpret_cast<f32x4 *>(&t[k][c]) = v[j];
-            }
+    DEVI void store(Tile &t, int tid) const {
+        int r, c;
+        if (!place(tid, r, c)) return;
+        const X3 v = split_chunk(x);
+        const int slot = c * Shape::P + r;
+        t.p[0][slot] = __builtin_bit_cast(u32x4, v.h);
+        t.p[1][slot] = __builtin_bit_cast(u32x4, v.m);
+        t.p[2][slot] = __builtin_bit_cast(u32x4, v.l);
+    }
+    // The MFMA operand of rows row0 + (l % 32): k in the order {4g..4g+3, 8+4g..8+4g+3} (g = l / 32),
+    // which is what a transposed read gives.
+    DEVI static uint32_t lanebase(int lane) {
+        if constexpr (ALONG_K) return (uint32_t)((lane & 31) * 16 + (lane >> 5) * 8);
+        else return tr_lanebase<BK, R>(lane);
+    }
+    DEVI static bf16x8 plane(const u32x4 *t, uint32_t base, int row0) {
+        if constexpr (ALONG_K) {
+            const char *q = reinterpret_cast<const char *>(t) + base + row0 * 16;
+            const uint2 lo = *reinterpret_cast<const uint2 *>(q), hi = *reinterpret_cast<const uint2 *>(q + Shape::CS);
+            return __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y});
         } else {
-#pragma unroll
-            for (int j = 0; j < N; ++j) {
-                const int i = tid + kThreads * j, r = i % R, k = i / R;
-                t[k][r] = s[j];
-            }
+            return tr_frag<BK, R>(t, base, 0, row0 / 32);
         }
+    }
+    DEVI static X3 frag(const Tile &t, uint32_t base, int row0) {
+        return {plane(t.p[0], base, row0), plane(t.p[1], base, row0), plane(t.p[2], base, row0)};
     }
 };
 
-template <int BM, int BN, int LA, int LB, int BK>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BK == 16 ? 4 : 2, BK == 16 ? 4 : 2))) void bmm_f32_kernel(BmmArgs g) {
+// Three workgroups per CU, two where the 128 x 128 tile reads an operand transposed (their registers).
+constexpr int waves_per_simd(int BN, int LA, int LB) { return BN == 128 && (LA == CONTIG_MN || LB == CONTIG_MN) ? 2 : 3; }
+
+template <int BM, int BN, int LA, int LB>
+__global__ __launch_bounds__(kThreads)
+__attribute__((amdgpu_waves_per_eu(waves_per_simd(BN, LA, LB), waves_per_simd(BN, LA, LB)))) void bmm_f32_kernel(BmmArgs g) {
     constexpr int TM = BM / 64, TN = BN / 64;  // 32 x 32 MFMA tiles per wave along m, n
     static_assert(TM >= 1 && TN >= 1, "a wave covers at least 32 x 32");
-    __shared__ BmmSmem<BM, BN, BK> sm;
+    typedef Operand<BM, LA> OpA;
+    typedef Operand<BN, LB> OpB;
+    __shared__ typename OpA::Tile ta[2];
+    __shared__ typename OpB::Tile tb[2];
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, gh = lane >> 5;
-    const int wave = tid >> 6, wm = wave >> 1, wn = wave & 1;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
     const int mt = (g.m + BM - 1) / BM, nt = (g.n + BN - 1) / BN, per = mt * nt;
     // The tiles of one batch item run on one XCD (workgroup w goes to XCD w % 8), so its A and B
     // panels are read from one L2.
@@ -132,15 +142,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BK == 
         return kt;
     };
 
-    Stage<BM, LA, BK> sa;
-    Stage<BN, LB, BK> sb;
-    int kt = next_live(0);
+    OpA sa;
+    OpB sb;
+    const int first = next_live(0);
+    int kt = first;
     // B's "rows" are its n columns: its row stride is the n stride, its k stride the k stride.
-    sa.load(ap, g.sam, g.sak, m0, g.m, kt * BK, kk, tid);
-    sb.load(bp, g.sbn, g.sbk, n0, g.n, kt * BK, kk, tid);
-    sa.store(sm.a[0], tid);
-    sb.store(sm.b[0], tid);
-    __syncthreads();
+    auto load = [&](int t) {
+        sa.load(ap, g.sam, g.sak, m0, g.m, t * BK, kk, tid);
+        sb.load(bp, g.sbn, g.sbk, n0, g.n, t * BK, kk, tid);
+    };
+    load(kt);
+    sa.store(ta[0], tid);
+    sb.store(tb[0], tid);
+    int next = next_live(kt + 1);
+    if (next < nk) load(next);
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -150,32 +165,58 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(BK == 
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
 
+    const uint32_t abase = OpA::lanebase(lane), bbase = OpB::lanebase(lane);
     for (int buf = 0; kt < nk; buf ^= 1) {
-        const int next = next_live(kt + 1);
-        if (next < nk) {
-            sa.load(ap, g.sam, g.sak, m0, g.m, next * BK, kk, tid);
-            sb.load(bp, g.sbn, g.sbk, n0, g.n, next * BK, kk, tid);
-        }
-        const float(*ta)[BM + kPad] = sm.a[buf];
-        const float(*tb)[BN + kPad] = sm.b[buf];
+        __syncthreads();  // tile kt is in LDS; everyone is done with the one before
+        X3 fa[TM], fb[TN];
 #pragma unroll
-        for (int k = 0; k < BK; k += 2) {
-            float fa[TM], fb[TN];
+        for (int i = 0; i < TM; ++i) fa[i] = OpA::frag(ta[buf], abase, wm * (BM / 2) + 32 * i);
 #pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = ta[k + gh][wm * (BM / 2) + 32 * i + lr];
+        for (int j = 0; j < TN; ++j) fb[j] = OpB::frag(tb[buf], bbase, wn * (BN / 2) + 32 * j);
 #pragma unroll
-            for (int j = 0; j < TN; ++j) fb[j] = tb[k + gh][wn * (BN / 2) + 32 * j + lr];
+        for (int t = 0; t < 6; ++t)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = mfma_f32(fa[i], fb[j], acc[i][j]);
-        }
+                for (int j = 0; j < TN; ++j) acc[i][j] = mfma_x3_part(fa[i], fb[j], acc[i][j], t);
         if (next < nk) {
-            sa.store(sm.a[buf ^ 1], tid);
-            sb.store(sm.b[buf ^ 1], tid);
+            sa.store(ta[buf ^ 1], tid);
+            sb.store(tb[buf ^ 1], tid);
         }
-        __syncthreads();
         kt = next;
+        next = next_live(kt + 1);
+        if (next < nk) load(next);
+    }
+
+    // Sums that are not finite again in plain float32: an infinite element may have met NaN
+    // remainders (x3.hpp).
+    float bad = 0.f;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) bad += not_finite(acc[i][j]);
+    if (__any(bad != 0.f)) {
+        for (int i = 0; i < TM; ++i)
+            for (int j = 0; j < TN; ++j) {
+                const int col = min(n0 + wn * (BN / 2) + 32 * j + lr, g.n - 1);
+                f32x16 t;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) t[e] = 0.f;
+                for (int q = first; q < nk; q = next_live(q + 1))
+                    for (int k = q * BK; k < min((q + 1) * BK, kk); ++k) {
+                        const float b = bp[col * g.sbn + k * g.sbk];
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            const int row = min(m0 + wm * (BM / 2) + 32 * i + acc_row(e, gh), g.m - 1);
+                            t[e] = fmaf(ap[row * g.sam + k * g.sak], b, t[e]);
+                        }
+                    }
+#pragma unroll
+                for (int ii = 0; ii < TM; ++ii)
+#pragma unroll
+                    for (int jj = 0; jj < TN; ++jj)
+                        if (ii == i && jj == j) acc[ii][jj] = t;
+            }
     }
 
     float *cp = g.c + (int64_t)bt * g.scb;
@@ -212,27 +253,21 @@ int layout_b(const BmmArgs &g) {
     return SCALAR;
 }
 
-template <int BM, int BN, int LA, int BK>
+template <int BM, int BN, int LA>
 hipError_t launch_b(const BmmArgs &g, int lb, dim3 grid, hipStream_t st) {
-    if (lb == CONTIG_K) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_K, BK>, grid, dim3(kThreads), st, g);
-    if (lb == CONTIG_MN) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_MN, BK>, grid, dim3(kThreads), st, g);
-    return launch(bmm_f32_kernel<BM, BN, LA, SCALAR, BK>, grid, dim3(kThreads), st, g);
+    if (lb == CONTIG_K) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_K>, grid, dim3(kThreads), st, g);
+    if (lb == CONTIG_MN) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_MN>, grid, dim3(kThreads), st, g);
+    return launch(bmm_f32_kernel<BM, BN, LA, SCALAR>, grid, dim3(kThreads), st, g);
 }
 
-template <int BM, int BN, int BK>
-hipError_t launch_k(const BmmArgs &g, hipStream_t st) {
+template <int BM, int BN>
+hipError_t launch_t(const BmmArgs &g, hipStream_t st) {
     const int64_t tiles = (int64_t)((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN) * g.batch;
     const dim3 grid((unsigned)tiles);
     const int la = layout_a(g), lb = layout_b(g);
-    if (la == CONTIG_K) return launch_b<BM, BN, CONTIG_K, BK>(g, lb, grid, st);
-    if (la == CONTIG_MN) return launch_b<BM, BN, CONTIG_MN, BK>(g, lb, grid, st);
-    return launch_b<BM, BN, SCALAR, BK>(g, lb, grid, st);
-}
-
-// BK = 16 (four workgroups per CU) unless the causal mode trims k per tile.
-template <int BM, int BN>
-hipError_t launch_t(const BmmArgs &g, hipStream_t st) {
-    return g.causal_mode >= 2 ? launch_k<BM, BN, 32>(g, st) : launch_k<BM, BN, 16>(g, st);
+    if (la == CONTIG_K) return launch_b<BM, BN, CONTIG_K>(g, lb, grid, st);
+    if (la == CONTIG_MN) return launch_b<BM, BN, CONTIG_MN>(g, lb, grid, st);
+    return launch_b<BM, BN, SCALAR>(g, lb, grid, st);
 }
 
 // Zeroes C when k == 0 (the reference returns zeros); C is (batch, m, n) through its strides.

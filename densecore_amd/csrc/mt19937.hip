@@ -257,8 +257,7 @@ __global__ __launch_bounds__(256) void mt_base_kernel(MtArgs a) {
 // partial windows are XORed, and the workgroups' ones stand side by side in dst (`src_split` of
 // them in src), XORed by whoever reads them.
 // Bound: VALU (about 6 M XORs per jump) and, in a launch of few jumps, one workgroup's latency, so
-// the level-1 jumps (at most 64) are split over 8 workgroups each: 98 -> 1L us for the 6 of 25 M
-// draws.  The sequence is 20576 words, 96 more than half of a CU's LDS: its last words are made
+// the level-1 jumps (at most 64) are split over 8 workgroups each.  The sequence is 20576 words, 96 more than half of a CU's LDS: its last words are made
 // after the terms that read the first ones are summed, in their place, and two workgroups share a
 // CU.  Both launches for 25 M draws (6 level-1, 384 level-0 jumps): 300 -> 143 us.
 constexpr int kSeqWords = 20480;  // LDS: half a CU's
