@@ -595,7 +595,7 @@ constexpr int kX3Threads = 2 * kThreads;
 
 template <int D>
 struct alignas(16) BwdSmemX3 {
-    X3Tile<kBM, D> q[3], o[2];       // at a tile's start the K, then V rows of the first four waves' keys
+    X3Tile<kBM, D> q[3], o[2];
     float p[kWaves][16][64];         // P, accumulator registers by lane
     X3Tile<32, 32> ds[kWaves];       // dS: rows are keys, columns the step's queries
     float part[kWaves][kBM][D + 4];  // a wave's share of dQ
@@ -713,16 +713,24 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             stage.store(sm.o[buf], gtid);
             sm.lse[buf][gtid & (kBM - 1)] = lse_next, sm.dsum[buf][gtid & (kBM - 1)] = dsum_next;
         };
-        // The keys' rows, through LDS tiles (waves w and w + 4 share tile w): K as A's row operand and
-        // B's transposed one, then V as B's row operand.
+        // The keys' rows, through LDS tiles where dS and the dQ shares will be (waves w and w + 4 share
+        // tile w): K as A's row operand and B's transposed one, then V as B's row operand.  The first
+        // steps' Q and dO are on their way meanwhile.
         X3 kv[KSTEP], kT[NDT][2];
         {
-            X3Tile<kBM, D> &wt = wave < 3 ? sm.q[wave] : sm.o[0];
+            static_assert(kWaves * sizeof(X3Tile<kBM, D>) <= sizeof(sm.ds) + sizeof(sm.part), "the rows fit");
+            X3Tile<kBM, D> &wt = reinterpret_cast<X3Tile<kBM, D> *>(&sm.ds[0])[wave];
             X3Stage<kBM, D, 64, VEC> rows;
             rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, lane);
             load_step();
             __syncthreads();  // a previous tile's last readers of these areas are done
-            if (group_a) rows.store(wt, lane);
+            if (group_a) {
+                rows.store(wt, lane);
+                store_do(0);
+            } else {
+                stage.store(sm.q[0], gtid);
+            }
+            if (i0 + 1 < i1) load_step();
             __syncthreads();
             if (group_a) {
 #pragma unroll
@@ -739,18 +747,10 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int st = 0; st < KSTEP; ++st) kv[st] = row_frag_x3(wt, rowb, 0, st);
-            }
-            __syncthreads();
-        }
-        if (group_a) {
-            store_do(0);
-            if (i0 + 1 < i1) load_step();
-        } else {
-            stage.store(sm.q[0], gtid);
-            if (i0 + 1 < i1) {
-                load_step();
-                stage.store(sm.q[1], gtid);
-                if (i0 + 2 < i1) load_step();
+                if (i0 + 1 < i1) {
+                    stage.store(sm.q[1], gtid);
+                    if (i0 + 2 < i1) load_step();
+                }
             }
         }
         __syncthreads();  // Q of the first two steps, dO of the first
@@ -1486,8 +1486,10 @@ __global__ __launch_bounds__(256) void bwd_reduce_f32_kernel(BwdArgs a, StreamK 
     }
 }
 
-// Workgroups of the backward that fit on the device at once (the occupancy bwd_waves_per_eu sets:
-// two per CU at D <= 64 without a mask, one otherwise); 0 if unknown.
+// The slots the schedules below were measured on: two workgroups per CU at D <= 64 without a mask,
+// one otherwise; 0 if unknown.  (key_tile_x3 runs one per CU at every D <= 64; the lines between the
+// schedules hold for it too, but it is given one range per CU: two cost a second prologue each,
+// causal B5 H16 L241 D64 61.8 against 51.5 us, B1 H12 L521 62.0 against 43.7.)
 int resident_workgroups(int D, bool mask) { return device_cus() * (D <= 64 && !mask ? 2 : 1); }
 
 // The stream-K schedule where whole tiles leave part of the device idle (measured on one MI355X,
@@ -1512,7 +1514,7 @@ StreamK plan_streamk(const AttnShape &s, int D, bool mask) {
     const int64_t last = tiles % slots;  // workgroups of the last, partial wave
     const bool underfilled = s.causal ? tiles <= slots : tiles < slots;
     const bool ragged = !s.causal && tiles < 4 * (int64_t)slots && last > 0 && 4 * last <= 3 * (int64_t)slots;
-    if (underfilled || ragged) k.chunks = slots;
+    if (underfilled || ragged) k.chunks = D <= 64 ? std::max(device_cus() & ~7, 8) : slots;
     return k;
 }
 
