@@ -40,6 +40,7 @@
 #include "common.hpp"
 #include "fwd_split.hpp"
 #include "params.hpp"
+#include "row_mask.hpp"
 #include "tile_bf16.hpp"
 
 namespace dc {
@@ -149,11 +150,12 @@ __host__ __device__ inline int dkdv_pieces(const AttnShape &s, int kt, int chunk
     return n > 1 ? n : 1;
 }
 
-template <int D, bool CAUSAL, bool MASK, bool VEC, bool F16, bool SPLIT = false>
+template <int D, bool CAUSAL, MaskKind MASK, bool VEC, bool F16, bool SPLIT = false>
 __global__ __launch_bounds__(KLayout<D>::THREADS) void bwd_dkdv_bf16_kernel(BwdArgs a) {
     constexpr int KSTEP = D / 16, NDT = D / 32;
     constexpr int KW = KLayout<D>::W, KN = KLayout<D>::N, QB = KLayout<D>::QB;
     static_assert(!SPLIT || KN == kKN, "split grids are planned over 128-key tiles");
+    constexpr bool ROW = MASK == kRowMask;
     __shared__ DkdvSmem<D> sm;
 
     const AttnShape &s = a.s;
@@ -163,6 +165,7 @@ __global__ __launch_bounds__(KLayout<D>::THREADS) void bwd_dkdv_bf16_kernel(BwdA
     const int nkt = (s.S + KN - 1) / KN;
     const int w = logical_block();
     int bhk = w / nkt, kt_ = w % nkt;  // causal: small n0 (most queries) first
+    if (ROW && !dealt_block(s.B * s.Hkv, nkt, w, &bhk, &kt_)) return;
     // Split: blocks run over (kv head, key tile, piece), the pieces of a key tile adjacent.
     int piece = 0, npieces = 1;
     if constexpr (SPLIT) {
@@ -246,9 +249,13 @@ __global__ __launch_bounds__(KLayout<D>::THREADS) void bwd_dkdv_bf16_kernel(BwdA
 #pragma unroll
         for (int r = 0; r < 16; ++r) dk[dt][r] = 0.f, dv[dt][r] = 0.f;
 
+    float mkey = 0.f;
     for (int i = i_begin; i < nsteps; ++i) {
         const int bh = step_bh(i), h = bh - b * s.H, m0 = step_m0(i), buf = i % QB;
         RowRaw stat = {0.f, false};
+        // A row mask's value for this lane's key, once per head, ahead of the transfers below.
+        if (ROW && (i == i_begin || i % per_head == 0))
+            mkey = key < s.S ? s.mask[(int64_t)b * s.msb + (int64_t)h * s.msh + key] : 0.f;
         if constexpr (QB == 2) {
             if (VEC) wait_vmem();
             __syncthreads();  // step i's tiles landed (and K/V at i = 0); step i - 1 is done
@@ -267,7 +274,7 @@ __global__ __launch_bounds__(KLayout<D>::THREADS) void bwd_dkdv_bf16_kernel(BwdA
 
         const int mq = m0 + 32 * qh;  // this wave's 32 queries
         const u32x4 *qt = sm.m.q[buf], *ot = sm.m.o[buf];
-        const float *mbase = MASK ? s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh : nullptr;
+        const float *mbase = MASK == kFullMask ? s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh : nullptr;
         const bool live = kw0 < s.S && mq < s.L && (!CAUSAL || mq + 31 >= kw0);
         if (live) {
             // dP accumulates onto -dsum, so the MFMAs leave dP - dsum.  The rows' -lse log2 e are
@@ -323,7 +330,7 @@ __global__ __launch_bounds__(KLayout<D>::THREADS) void bwd_dkdv_bf16_kernel(BwdA
                         // exponent in base 2: scale q.k (+ mask) - lse, times log2 e
                         float x;
                         if (MASK) {
-                            const float mk = (qq < s.L && key < s.S) ? mbase[(int64_t)qq * s.msl + key] : 0.f;
+                            const float mk = ROW ? mkey : (qq < s.L && key < s.S) ? mbase[(int64_t)qq * s.msl + key] : 0.f;
                             x = fmaf(fmaf(sacc[r], sc, mk), kLog2e, nl[r4][j]);
                         } else {
                             x = fmaf(sacc[r], sc_log2, nl[r4][j]);
@@ -465,17 +472,22 @@ struct alignas(16) DqSmem {
 // take 136 KB of LDS and its Q, dO and dQ registers 256 per lane: one workgroup, one wave per SIMD.
 constexpr int dq_waves_per_eu(int D) { return D > 128 ? 1 : 2; }
 
-template <int D, bool CAUSAL, bool MASK, bool VEC, bool F16, bool SPLIT = false>
+template <int D, bool CAUSAL, MaskKind MASK, bool VEC, bool F16, bool SPLIT = false>
 __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_waves_per_eu(D), dq_waves_per_eu(D)))) void bwd_dq_bf16_kernel(BwdArgs a) {
     constexpr int KSTEP = D / 16, NDT = D / 32, NT = kQN / 32;
+    constexpr bool ROW = MASK == kRowMask;
+    static_assert(kQN == 64, "a row mask's tile is one value per lane");
     __shared__ DqSmem<D> sm;
+    __shared__ float row_values[ROW ? kQW : 1][64];
 
     const AttnShape &s = a.s;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nqt = (s.L + kQM - 1) / kQM;
     const int w = logical_block();
-    int bh = w / nqt, qt = CAUSAL ? nqt - 1 - w % nqt : w % nqt;
+    int bh = w / nqt, qt = w % nqt;
+    if (ROW && !dealt_block(s.B * s.H, nqt, w, &bh, &qt)) return;
+    if (CAUSAL) qt = nqt - 1 - qt;
     // Split: blocks run over (head, query tile longest first, piece) (fwd_split.hpp).
     int piece = 0, npieces = 1;
     if constexpr (SPLIT) {
@@ -523,7 +535,8 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
     float dsum_q = qi < s.L ? a.dsum[(int64_t)bh * s.L + qi] : 0.f;
     if constexpr (F16) dsum_q = ldexpf(dsum_q, fs.e_pv);
     const float *mrow = nullptr;
-    if (MASK) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh + (int64_t)qi * s.msl;
+    if (ROW) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh;
+    else if (MASK) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh + (int64_t)qi * s.msl;
 
     f32x16 dq[NDT];
 #pragma unroll
@@ -536,28 +549,44 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
     // This block's key tiles [t_begin, ntiles): all of them, or its piece's.
     const int t_begin = SPLIT ? piece * all_tiles / npieces : 0;
     const int ntiles = SPLIT ? (piece + 1) * all_tiles / npieces : all_tiles;
-    auto fill = [&](int t) {
+    // Tile t goes to buffer i & 1 (the i-th visited); a row mask's dead tiles are not visited.
+    auto fill = [&](int i, int t) {
         const int n0 = t * kQN, rows = min(kQN, s.S - n0);
-        fill_cm<kQN, D, VEC, kQW>(sm.k[t & 1], kb + (int64_t)n0 * s.E, rows, s.E, wave, lane);
-        fill_cm<kQN, D, VEC, kQW>(sm.v[t & 1], vb + (int64_t)n0 * s.E, rows, s.E, wave, lane);
+        fill_cm<kQN, D, VEC, kQW>(sm.k[i & 1], kb + (int64_t)n0 * s.E, rows, s.E, wave, lane);
+        fill_cm<kQN, D, VEC, kQW>(sm.v[i & 1], vb + (int64_t)n0 * s.E, rows, s.E, wave, lane);
     };
-    if (t_begin < ntiles) fill(t_begin);
+    LiveTiles tiles(mrow, s.S, ntiles, lane);
+    int t0 = t_begin;
+    if constexpr (ROW) t0 = tiles.next(0);
+    float mcur = ROW ? tiles.value(t0) : 0.f;
+    if (t0 < ntiles) fill(0, t0);
     const uint32_t rowb = row_lanebase<kQN, D>(lane);
     const uint32_t trb = tr_lanebase<kQN, D>(lane);
 
-    for (int t = t_begin; t < ntiles; ++t) {
+    for (int i = 0, t = t0, tnext; t < ntiles; ++i, t = tnext) {
+        tnext = ROW ? tiles.next(t + 1) : t + 1;
         const int n0 = t * kQN;
         if (VEC) wait_vmem();
         __syncthreads();
-        if (t + 1 < ntiles) fill(t + 1);
-        const u32x4 *kt_ = sm.k[t & 1], *vt_ = sm.v[t & 1];
+        uint64_t open = 0;  // row mask: this tile's keys that are not masked
+        if constexpr (ROW) {
+            open = __ballot(mcur != -INFINITY);
+            row_values[wave][lane] = mcur;  // read back by this wave alone
+            mcur = tiles.value(tnext);
+        }
+        if (tnext < ntiles) fill(i + 1, tnext);
+        const u32x4 *kt_ = sm.k[i & 1], *vt_ = sm.v[i & 1];
 
         bool live[NT];
 #pragma unroll
         for (int kt = 0; kt < NT; ++kt)
             live[kt] = (n0 + kt * 32 < s.S) && (!CAUSAL || n0 + kt * 32 <= wave_last_q);
-        float mv[MASK ? NT : 1][16];
-        if constexpr (MASK) {
+        float mv[MASK == kFullMask ? NT : 1][16];
+        if constexpr (ROW) {
+#pragma unroll
+            for (int kt = 0; kt < NT; ++kt) live[kt] = live[kt] && (uint32_t)(open >> (32 * kt)) != 0;
+        }
+        if constexpr (MASK == kFullMask) {
 #pragma unroll
             for (int kt = 0; kt < NT; ++kt) {
                 bool any_open = false;
@@ -582,6 +611,13 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
             // per SIMD pass the same barriers, measured no difference).
             __builtin_amdgcn_s_setprio(1);
             f32x16 sacc, pacc;
+            f32x4 mrk[4];  // the row mask at this lane's keys, read ahead of the products' operands
+            if constexpr (ROW) {
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4)
+                    mrk[r4] = *reinterpret_cast<const f32x4 *>(&row_values[wave][32 * kt + 8 * r4 + 4 * g]);
+                __builtin_amdgcn_sched_barrier(0);  // keep these reads out of the MFMA schedule below
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) sacc[r] = 0.f, pacc[r] = 0.f;
 #pragma unroll
@@ -594,14 +630,14 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
             __builtin_amdgcn_sched_barrier(0);
             __builtin_amdgcn_s_setprio(0);
             // K^T for dQ^T += K^T dS^T, one 16-key half u at a time.  Without a mask both halves
-            // are read here, while dS^T is formed; the masked kernels (whose mask values take 32
-            // more registers) read each just before its products.
+            // are read here, while dS^T is formed, and with a row mask too; full masks (whose values
+            // take 32 more registers) read each just before its products.
             bf16x8 fa[2][NDT];
             auto load_fa = [&](int u) {
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt) fa[u][dt] = tr_frag<kQN, D>(kt_, trb, 32 * kt + 16 * u, dt);
             };
-            if constexpr (!MASK) load_fa(0), load_fa(1);
+            if constexpr (MASK != kFullMask) load_fa(0), load_fa(1);
             // dS^T; EDGE (keys past S or past the diagonal) is a separate instantiation so
             // that the common path carries no per-element masking.  pm[u]: the largest P 2^-24
             // of the 16-key half u, as bits (P >= 0 orders as an unsigned integer); where some P
@@ -613,7 +649,8 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
                 for (int r = 0; r < 16; ++r) {
                     // exponent in base 2: scale q.k (+ mask) - lse, times log2 e
                     float x;
-                    if (MASK) x = fmaf(fmaf(sacc[r], sc, mv[kt][r]), kLog2e, nlse2);
+                    if (MASK == kFullMask) x = fmaf(fmaf(sacc[r], sc, mv[kt][r]), kLog2e, nlse2);
+                    else if (ROW) x = fmaf(fmaf(sacc[r], sc, mrk[r >> 2][r & 3]), kLog2e, nlse2);
                     else x = fmaf(sacc[r], sc_log2, nlse2);
                     if (EDGE) {
                         const int key = n0 + kt * 32 + acc_row(r, g);
@@ -638,7 +675,7 @@ __global__ __launch_bounds__(kQThreads) __attribute__((amdgpu_waves_per_eu(dq_wa
                 } else {
                     split_bf16(sacc, 8 * u, sh, sl);
                 }
-                if constexpr (MASK) load_fa(u);
+                if constexpr (MASK == kFullMask) load_fa(u);
 #pragma unroll
                 for (int dt = 0; dt < NDT; ++dt) dq[dt] = mfma16<F16>(fa[u][dt], sh, dq[dt]);
                 if (!F16 || lo) {
@@ -751,7 +788,7 @@ BwdSplitPlan plan_bwd(const AttnShape &s) {
     const int nkt = (s.S + kKN - 1) / kKN;
     const int64_t BHk = (int64_t)s.B * s.Hkv;
     const int64_t slots_k = split_slots(
-        reinterpret_cast<const void *>(&bwd_dkdv_bf16_kernel<D, true, false, true, true, true>), kKThreads, nkt * BHk);
+        reinterpret_cast<const void *>(&bwd_dkdv_bf16_kernel<D, true, kNoMask, true, true, true>), kKThreads, nkt * BHk);
     if (slots_k > 0 && 2 * nkt * BHk <= slots_k) {
         int64_t steps = 0;
         int most = 0;
@@ -773,7 +810,7 @@ BwdSplitPlan plan_bwd(const AttnShape &s) {
     }
     const int64_t nqt = (s.L + kQM - 1) / kQM;
     const int64_t slots_q = split_slots(
-        reinterpret_cast<const void *>(&bwd_dq_bf16_kernel<D, true, false, true, true, true>), kQThreads,
+        reinterpret_cast<const void *>(&bwd_dq_bf16_kernel<D, true, kNoMask, true, true, true>), kQThreads,
         nqt * s.B * s.H);
     const FwdSplitPlan q = plan_split(s, kQM, kQN, slots_q);
     p.chunk_q = q.chunk, p.max_q = q.max_pieces, p.blocks_q = q.blocks;
@@ -792,44 +829,50 @@ hipError_t launch_split(const BwdArgs &args, const BwdSplitPlan &p, hipStream_t 
     const dim3 bk(kKThreads), bq(kQThreads), br(256);
     if (p.chunk_k > 0) {
         const dim3 gk((unsigned)p.blocks_k);
-        if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, false, VEC, true, true>, gk, bk, st, a));
-        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, false, VEC, true, true>, gk, bk, st, a));
+        if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, kNoMask, VEC, true, true>, gk, bk, st, a));
+        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, kNoMask, VEC, true, true>, gk, bk, st, a));
         const int64_t n = (int64_t)a.s.B * a.s.Hkv * a.s.S * ((a.s.E + 3) / 4);
         return_if(launch(bwd_split_reduce_kernel, dim3((unsigned)((n + 255) / 256)), br, st, a, 0));
     } else {
         const dim3 gk(((a.s.S + kKN - 1) / kKN) * a.s.B * a.s.Hkv);
-        if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, false, VEC, true>, gk, bk, st, a));
-        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, false, VEC, true>, gk, bk, st, a));
+        if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, kNoMask, VEC, true>, gk, bk, st, a));
+        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, kNoMask, VEC, true>, gk, bk, st, a));
     }
     if (p.chunk_q > 0) {
         const dim3 gq((unsigned)p.blocks_q);
-        if (causal) return_if(launch(bwd_dq_bf16_kernel<D, true, false, VEC, true, true>, gq, bq, st, a));
-        else return_if(launch(bwd_dq_bf16_kernel<D, false, false, VEC, true, true>, gq, bq, st, a));
+        if (causal) return_if(launch(bwd_dq_bf16_kernel<D, true, kNoMask, VEC, true, true>, gq, bq, st, a));
+        else return_if(launch(bwd_dq_bf16_kernel<D, false, kNoMask, VEC, true, true>, gq, bq, st, a));
         const int64_t n = (int64_t)a.s.B * a.s.H * a.s.L * ((a.s.E + 3) / 4);
         return launch(bwd_split_reduce_kernel, dim3((unsigned)((n + 255) / 256)), br, st, a, 1);
     }
     const dim3 gq(((a.s.L + kQM - 1) / kQM) * a.s.B * a.s.H);
-    if (causal) return launch(bwd_dq_bf16_kernel<D, true, false, VEC, true>, gq, bq, st, a);
-    return launch(bwd_dq_bf16_kernel<D, false, false, VEC, true>, gq, bq, st, a);
+    if (causal) return launch(bwd_dq_bf16_kernel<D, true, kNoMask, VEC, true>, gq, bq, st, a);
+    return launch(bwd_dq_bf16_kernel<D, false, kNoMask, VEC, true>, gq, bq, st, a);
 }
 
 template <int D, bool VEC, bool F16>
 hipError_t launch_dvf(const BwdArgs &a, hipStream_t st) {
-    const bool mask = a.s.mask != nullptr, causal = a.s.causal;
+    const bool mask = a.s.mask != nullptr, causal = a.s.causal, row = mask && a.s.msl == 0;
     constexpr int KN = KLayout<D>::N;
     const dim3 gk(((a.s.S + KN - 1) / KN) * a.s.B * a.s.Hkv), bk(KLayout<D>::THREADS);
     const dim3 gq(((a.s.L + kQM - 1) / kQM) * a.s.B * a.s.H), bq(kQThreads);
     if (a.s.S > 0) {
-        if (causal && mask) return_if(launch(bwd_dkdv_bf16_kernel<D, true, true, VEC, F16>, gk, bk, st, a));
-        else if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, false, VEC, F16>, gk, bk, st, a));
-        else if (mask) return_if(launch(bwd_dkdv_bf16_kernel<D, false, true, VEC, F16>, gk, bk, st, a));
-        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, false, VEC, F16>, gk, bk, st, a));
+        const dim3 gr(((a.s.S + KN - 1) / KN) * dealt_heads(a.s.B * a.s.Hkv));
+        if (causal && row) return_if(launch(bwd_dkdv_bf16_kernel<D, true, kRowMask, VEC, F16>, gr, bk, st, a));
+        else if (row) return_if(launch(bwd_dkdv_bf16_kernel<D, false, kRowMask, VEC, F16>, gr, bk, st, a));
+        else if (causal && mask) return_if(launch(bwd_dkdv_bf16_kernel<D, true, kFullMask, VEC, F16>, gk, bk, st, a));
+        else if (causal) return_if(launch(bwd_dkdv_bf16_kernel<D, true, kNoMask, VEC, F16>, gk, bk, st, a));
+        else if (mask) return_if(launch(bwd_dkdv_bf16_kernel<D, false, kFullMask, VEC, F16>, gk, bk, st, a));
+        else return_if(launch(bwd_dkdv_bf16_kernel<D, false, kNoMask, VEC, F16>, gk, bk, st, a));
     }
     if (a.s.L > 0) {
-        if (causal && mask) return_if(launch(bwd_dq_bf16_kernel<D, true, true, VEC, F16>, gq, bq, st, a));
-        else if (causal) return_if(launch(bwd_dq_bf16_kernel<D, true, false, VEC, F16>, gq, bq, st, a));
-        else if (mask) return_if(launch(bwd_dq_bf16_kernel<D, false, true, VEC, F16>, gq, bq, st, a));
-        else return_if(launch(bwd_dq_bf16_kernel<D, false, false, VEC, F16>, gq, bq, st, a));
+        const dim3 gr(((a.s.L + kQM - 1) / kQM) * dealt_heads(a.s.B * a.s.H));
+        if (causal && row) return_if(launch(bwd_dq_bf16_kernel<D, true, kRowMask, VEC, F16>, gr, bq, st, a));
+        else if (row) return_if(launch(bwd_dq_bf16_kernel<D, false, kRowMask, VEC, F16>, gr, bq, st, a));
+        else if (causal && mask) return_if(launch(bwd_dq_bf16_kernel<D, true, kFullMask, VEC, F16>, gq, bq, st, a));
+        else if (causal) return_if(launch(bwd_dq_bf16_kernel<D, true, kNoMask, VEC, F16>, gq, bq, st, a));
+        else if (mask) return_if(launch(bwd_dq_bf16_kernel<D, false, kFullMask, VEC, F16>, gq, bq, st, a));
+        else return_if(launch(bwd_dq_bf16_kernel<D, false, kNoMask, VEC, F16>, gq, bq, st, a));
     }
     return hipSuccess;
 }

@@ -12,7 +12,7 @@
 // and NaN values convert to themselves and do not set the scale.  The kernels fold 2^-e back
 // into the scalars they already multiply by.
 //
-// Two passes: slab_max_kernel reduces each of `parts` segments (of `per` elements) of a slab to
+// Short slabs take one launch (slab_one_pass_kernel).  Longer ones two passes: slab_max_kernel reduces each of `parts` segments (of `per` elements) of a slab to
 // its largest finite magnitude; slab_convert_kernel reads a slab's partial maxima, derives e
 // (written once per slab) and converts its segment.  Each pass is one launch for all the
 // tensors a call copies (the backward's four): its blocks are dealt to the tensors in order.
@@ -145,6 +145,50 @@ __global__ __launch_bounds__(kThreads) void slab_convert_kernel(SlabJobs J) {
     }
 }
 
+// Slabs of at most kOnePass elements: one workgroup keeps a slab in registers between its maximum
+// and its conversion, so it is read once and the call is one launch (B16 H12 L512 E64, four
+// tensors: 22.8 us against 17.9 + 11.2 in two passes; B3 H6 L84: forward 21.5 -> 18.8 us).  Longer slabs would leave too few workgroups.
+constexpr int kOneThreads = 1024, kOneVecs = 8;
+constexpr int64_t kOnePass = (int64_t)8 * kOneThreads * kOneVecs;
+
+__global__ __launch_bounds__(kOneThreads) void slab_one_pass_kernel(SlabJobs J) {
+    int s;
+    const int j = job_of(J, (int)blockIdx.x, &s);
+    const int slab = (int)J.slab[j];
+    const uint16_t *x = J.src[j] + (int64_t)s * slab;
+    u16x8 v[kOneVecs];
+    float m = 0.f;
+#pragma unroll
+    for (int u = 0; u < kOneVecs; ++u) {
+        const int i = 8 * (u * kOneThreads + (int)threadIdx.x);
+        v[u] = i < slab ? load_nt(reinterpret_cast<const u16x8 *>(x + i)) : u16x8{0, 0, 0, 0, 0, 0, 0, 0};
+    }
+#pragma unroll
+    for (int u = 0; u < kOneVecs; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) m = fmaxf(m, finite_abs(v[u][e]));
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
+    __shared__ float wm[kOneThreads / 64];
+    if ((threadIdx.x & 63) == 0) wm[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kOneThreads / 64; ++w) m = fmaxf(m, wm[w]);
+    const int e = slab_exp(m);
+    if (threadIdx.x == 0) J.exps[j][s] = e;
+    _Float16 *y = J.dst[j] + (int64_t)s * slab;
+#pragma unroll
+    for (int u = 0; u < kOneVecs; ++u) {
+        const int i = 8 * (u * kOneThreads + (int)threadIdx.x);
+        if (i >= slab) continue;
+        f16x8 o;
+#pragma unroll
+        for (int c = 0; c < 8; ++c)
+            o[c] = static_cast<_Float16>(ldexpf(__uint_as_float((uint32_t)v[u][c] << 16), e));
+        *reinterpret_cast<f16x8 *>(y + i) = o;
+    }
+}
+
 }  // namespace
 
 // Segment length for `nslabs` slabs of `slab` elements: a multiple of 2048 (8 elements per
@@ -195,6 +239,12 @@ hipError_t launch_to_f16(const F16Copy *copies, int n, int64_t nslabs, float *pa
         ++J.n;
     }
     if (J.n == 0) return hipSuccess;
+    bool one = true;
+    for (int j = 0; j < J.n; ++j) one = one && J.slab[j] <= kOnePass && J.vec[j];
+    if (one) {  // a workgroup per slab
+        for (int j = 0; j < J.n; ++j) J.first[j + 1] = J.first[j] + (int)nslabs;
+        return launch(slab_one_pass_kernel, dim3((unsigned)J.first[J.n]), dim3(kOneThreads), st, J);
+    }
     const dim3 grid((unsigned)J.first[J.n]), block(kThreads);
     return_if(launch(slab_max_kernel, grid, block, st, J));
     return launch(slab_convert_kernel, grid, block, st, J);

@@ -26,6 +26,7 @@
 #include "common.hpp"
 #include "fwd_split.hpp"
 #include "params.hpp"
+#include "row_mask.hpp"
 #include "tile_bf16.hpp"
 
 namespace dc {
@@ -56,12 +57,15 @@ DEVI void fill_tile(KVTileBf16<D> &t, const __bf16 *kb, const __bf16 *vb, int n0
 // per CU and one wave per SIMD (512 registers).
 constexpr int fwd_waves_per_eu(int D) { return D > 128 ? 1 : 2; }
 
-template <int D, bool CAUSAL, bool MASK, bool VEC>
+template <int D, bool CAUSAL, MaskKind MASK, bool VEC>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_waves_per_eu(D), fwd_waves_per_eu(D)))) void fwd_bf16_kernel(FwdArgs a) {
     constexpr int NT = kBN / 32;  // 32-key sub-tiles per tile
     constexpr int KSTEP = D / 16; // MFMA k-steps over the head dim
     constexpr int NDT = D / 32;   // 32-dim output tiles
+    constexpr bool ROW = MASK == kRowMask;
+    static_assert(kBN == 64, "a row mask's tile is one value per lane");
     __shared__ KVTileBf16<D> sm[2];
+    __shared__ float row_values[ROW ? kThreads / 64 : 1][64];
 
     const AttnShape &s = a.s;
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, g = lane >> 5;
@@ -70,7 +74,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
     const int nblk = gridDim.x;
     int w = blockIdx.x;
     if ((nblk & 7) == 0) w = (w & 7) * (nblk >> 3) + (w >> 3);
-    const int bh = w / nqt, qt = CAUSAL ? nqt - 1 - w % nqt : w % nqt;
+    int bh = w / nqt, qt = w % nqt;
+    if (ROW && !dealt_block(s.B * s.H, nqt, w, &bh, &qt)) return;
+    if (CAUSAL) qt = nqt - 1 - qt;
     const int b = bh / s.H, h = bh % s.H, hk = h / s.repeat;
     const int q0 = qt * kBM;
     const int qi = q0 + wave * 32 + lr;  // this lane's query
@@ -108,7 +114,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
         }
     }
     const float *mrow = nullptr;
-    if (MASK) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh + (int64_t)qi * s.msl;
+    if (ROW) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh;
+    else if (MASK) mrow = s.mask + (int64_t)b * s.msb + (int64_t)h * s.msh + (int64_t)qi * s.msl;
 
     f32x16 oacc[NDT];
 #pragma unroll
@@ -119,17 +126,28 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
 
     const int kv_end = CAUSAL ? min(q0 + kBM, s.S) : s.S;
     const int ntiles = (kv_end + kBN - 1) / kBN;
-    if (ntiles > 0) fill_tile<D, VEC>(sm[0], kb, vb, 0, s.S, s.E, wave, lane);
+    // Tile t goes to buffer i & 1 (the i-th visited); a row mask's dead tiles are not visited.
+    LiveTiles tiles(mrow, s.S, ntiles, lane);
+    int t0 = 0;
+    if constexpr (ROW) t0 = tiles.next(0);
+    float mcur = ROW ? tiles.value(t0) : 0.f;
+    if (t0 < ntiles) fill_tile<D, VEC>(sm[0], kb, vb, t0 * kBN, s.S, s.E, wave, lane);
 
     const uint32_t rowb = row_lanebase<kBN, D>(lane);
     const uint32_t trb = tr_lanebase<kBN, D>(lane);
 
-    auto tile = [&](int t) {
+    auto tile = [&](int i, int t, int tnext) {
         const int n0 = t * kBN;
-        KVTileBf16<D> &cur = sm[t & 1];
+        KVTileBf16<D> &cur = sm[i & 1];
         if (VEC) wait_vmem();  // this wave's transfers of tile t landed
         __syncthreads();       // everyone's landed; everyone is done with tile t - 1
-        if (t + 1 < ntiles) fill_tile<D, VEC>(sm[(t + 1) & 1], kb, vb, n0 + kBN, s.S, s.E, wave, lane);
+        uint64_t open = 0;  // row mask: this tile's keys that are not masked
+        if constexpr (ROW) {
+            open = __ballot(mcur != -INFINITY);
+            row_values[wave][lane] = mcur;  // read back by this wave alone
+            mcur = tiles.value(tnext);
+        }
+        if (tnext < ntiles) fill_tile<D, VEC>(sm[(i + 1) & 1], kb, vb, tnext * kBN, s.S, s.E, wave, lane);
 
         // K rows kt * 32 + (l % 32) for S^T; V^T (dims on lanes) for keys 16u + {4g..4g+3,
         // 8+4g..8+4g+3} of sub-tile kt, the rows P's accumulator registers 8u..8u+7 hold.
@@ -142,8 +160,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
             live[kt] = (n0 + kt * 32 < s.S) && (!CAUSAL || n0 + kt * 32 <= wave_last_q);
         // With a mask its values are read first; a sub-tile whose mask is -inf for every
         // (query, key) of the wave is skipped (its probabilities are exactly 0).
-        float mv[MASK ? NT : 1][16];
-        if constexpr (MASK) {
+        float mv[MASK == kFullMask ? NT : 1][16];
+        if constexpr (ROW) {
+#pragma unroll
+            for (int kt = 0; kt < NT; ++kt) live[kt] = live[kt] && (uint32_t)(open >> (32 * kt)) != 0;
+        }
+        if constexpr (MASK == kFullMask) {
 #pragma unroll
             for (int kt = 0; kt < NT; ++kt) {
                 bool any_open = false;
@@ -186,11 +208,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
             }
         }
 
-        if constexpr (MASK) {
+        if constexpr (MASK == kFullMask) {
 #pragma unroll
             for (int kt = 0; kt < NT; ++kt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) sacc[kt][r] = (sacc[kt][r] * s.scale + mv[kt][r]) * kLog2e;
+        } else if constexpr (ROW) {
+#pragma unroll
+            for (int kt = 0; kt < NT; ++kt)
+#pragma unroll
+                for (int r4 = 0; r4 < 4; ++r4) {
+                    const f32x4 m = *reinterpret_cast<const f32x4 *>(&row_values[wave][32 * kt + 8 * r4 + 4 * g]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        sacc[kt][4 * r4 + j] = (sacc[kt][4 * r4 + j] * s.scale + m[j]) * kLog2e;
+                }
         }
         if (edge) {
 #pragma unroll
@@ -248,7 +280,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(fwd_wa
             }
         }
     };
-    for (int t = 0; t < ntiles; ++t) tile(t);
+    for (int i = 0, t = t0; t < ntiles; ++i) {
+        const int tnext = ROW ? tiles.next(t + 1) : t + 1;
+        tile(i, t, tnext);
+        t = tnext;
+    }
 
     const float l_run = xor32_add(l_part);
     if (qi < s.L) {
@@ -580,20 +616,26 @@ FwdSplitPlan plan(const AttnShape &s) {
     return plan_split(s, kPPM, kBN, slots);
 }
 
+// The 4-wave kernel: masks, and head dims 129-256 with or without one.
+template <int D, bool VEC, bool CAUSAL>
+hipError_t launch_masked(const FwdArgs &a, hipStream_t st) {
+    const int nqt = (a.s.L + kBM - 1) / kBM, heads = a.s.B * a.s.H;
+    const dim3 block(kThreads);
+    if (a.s.mask && a.s.msl == 0)
+        return launch(fwd_bf16_kernel<D, CAUSAL, kRowMask, VEC>, dim3(nqt * dealt_heads(heads)), block, st, a);
+    if (a.s.mask) return launch(fwd_bf16_kernel<D, CAUSAL, kFullMask, VEC>, dim3(nqt * heads), block, st, a);
+    if constexpr (D > 128) return launch(fwd_bf16_kernel<D, CAUSAL, kNoMask, VEC>, dim3(nqt * heads), block, st, a);
+    else return hipErrorInvalidValue;  // not reached: the ping-pong kernel's
+}
+
 template <int D, bool VEC>
 hipError_t launch_dv(const FwdArgs &a, hipStream_t st) {
-    const bool mask = a.s.mask != nullptr;
     if constexpr (D > 128) {
         // Head dims 129-256: the 4-wave kernel, with or without a mask (the ping-pong kernel's
         // 8 waves would need more than 256 registers each); P enters P V as bf16 hi + lo.
-        const int nqt = (a.s.L + kBM - 1) / kBM;
-        const dim3 grid(nqt * a.s.B * a.s.H), block(kThreads);
-        if (a.s.causal && mask) return launch(fwd_bf16_kernel<D, true, true, VEC>, grid, block, st, a);
-        if (a.s.causal) return launch(fwd_bf16_kernel<D, true, false, VEC>, grid, block, st, a);
-        if (mask) return launch(fwd_bf16_kernel<D, false, true, VEC>, grid, block, st, a);
-        return launch(fwd_bf16_kernel<D, false, false, VEC>, grid, block, st, a);
+        return a.s.causal ? launch_masked<D, VEC, true>(a, st) : launch_masked<D, VEC, false>(a, st);
     } else {  // head dims up to 128 (the ping-pong kernel exists only there)
-        if (!mask) {
+        if (!a.s.mask) {
             const int nqt = (a.s.L + kPPM - 1) / kPPM;
             const dim3 grid(nqt * a.s.B * a.s.H), block(kPPThreads);
             if (a.v16) {
@@ -625,10 +667,7 @@ hipError_t launch_dv(const FwdArgs &a, hipStream_t st) {
             if (a.s.causal) return launch(fwd_bf16_pp_kernel<D, true, VEC, false>, grid, block, st, a);
             return launch(fwd_bf16_pp_kernel<D, false, VEC, false>, grid, block, st, a);
         }
-        const int nqt = (a.s.L + kBM - 1) / kBM;
-        const dim3 grid(nqt * a.s.B * a.s.H), block(kThreads);
-        if (a.s.causal) return launch(fwd_bf16_kernel<D, true, true, VEC>, grid, block, st, a);
-        return launch(fwd_bf16_kernel<D, false, true, VEC>, grid, block, st, a);
+        return a.s.causal ? launch_masked<D, VEC, true>(a, st) : launch_masked<D, VEC, false>(a, st);
     }
 }
 

@@ -30,6 +30,7 @@
 #include "fwd_order.hpp"
 #include "fwd_split.hpp"
 #include "params.hpp"
+#include "row_mask.hpp"
 #include "x3.hpp"
 
 namespace dc {
@@ -39,10 +40,6 @@ constexpr int kX3BN = 32;      // keys per tile
 constexpr int kX3Waves = 4;    // 32 queries each
 constexpr int kX3Threads = 64 * kX3Waves;
 constexpr int kX3M = 32 * kX3Waves;
-
-// kNoMask; kFullMask: a mask value per (query, key); kRowMask: the mask does not depend on the query
-// (stride 0 along L: key padding).
-enum MaskKind { kNoMask, kFullMask, kRowMask };
 
 // At D = 128 the queries' parts and the output take 160 registers and the tiles 110 KB of LDS: one
 // workgroup per CU, one wave per SIMD (two of single-buffered tiles: causal B2 H16 L2048 224 us
