@@ -216,13 +216,39 @@ __global__ __launch_bounds__(kThreads) void decode_split_kernel(DecodeArgs a) {
 template <typename T, int D>
 constexpr int kChunkKeys = group_chunk_keys(D, sizeof(T));
 
-DEVI f32x4 mfma_rows(f32x4 k, f32x4 q, f32x4 c) {
+// Sixteen keys' scores from a lane's N parts of their rows.  Float32: chains of two products of four
+// dims, summed in pairs as a tree (one chain through the accumulator: 1.5 to 3.5 times the error
+// against float64 of the split kernel, whose lanes sum their dims as a tree).  The barriers keep the
+// chains of one pair of parts in registers at a time.
+template <int I, int W, int N>
+DEVI f32x4 tree_rows(const f32x4 (&k)[N], const f32x4 (&q)[N]) {
+    if constexpr (W <= 2) {
+        f32x4 c[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) c = __builtin_amdgcn_mfma_f32_16x16x4f32(k[u], q[u], c, 0, 0, 0);
-    return c;
+        for (int u = 0; u < 4; ++u) c[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = I; i < I + W; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) c[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][u], q[i][u], c[u], 0, 0, 0);
+        const f32x4 t = (c[0] + c[1]) + (c[2] + c[3]);
+        __builtin_amdgcn_sched_barrier(0);
+        return t;
+    } else {
+        const f32x4 lo = tree_rows<I, W / 2>(k, q);
+        return lo + tree_rows<I + W / 2, W / 2>(k, q);
+    }
 }
-DEVI f32x4 mfma_rows(bf16x8 k, bf16x8 q, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(k, q, c, 0, 0, 0);
+template <int N>
+DEVI f32x4 mfma_rows(const f32x4 (&k)[N], const f32x4 (&q)[N]) {
+    static_assert((N & (N - 1)) == 0, "halved down to pairs");
+    return tree_rows<0, N>(k, q);
+}
+template <int N>
+DEVI f32x4 mfma_rows(const bf16x8 (&k)[N], const bf16x8 (&q)[N]) {
+    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < N; ++i) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k[i], q[i], c, 0, 0, 0);
+    return c;
 }
 
 template <typename T, int D, int HG, bool FULL>
@@ -297,11 +323,7 @@ __global__ __launch_bounds__(kThreads) void decode_group_kernel(DecodeArgs a) {
         }
         f32x4 sc[NG];
 #pragma unroll
-        for (int gi = 0; gi < NG; ++gi) {
-            sc[gi] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int i = 0; i < KS; ++i) sc[gi] = mfma_rows(kx[gi][i], qv[i], sc[gi]);
-        }
+        for (int gi = 0; gi < NG; ++gi) sc[gi] = mfma_rows(kx[gi], qv);
         // V's loads go out before the softmax: its latency hides part of theirs.
         vec_t vx[NV];
 #pragma unroll
@@ -340,16 +362,21 @@ __global__ __launch_bounds__(kThreads) void decode_group_kernel(DecodeArgs a) {
             __builtin_amdgcn_wave_barrier();
         }
         const float m_use = m_run == -INFINITY ? 0.f : m_run;
+        float l_chunk = 0.f;
 #pragma unroll
         for (int gi = 0; gi < NG; ++gi)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const float p = exp2_fast(sc[gi][r] - m_use);
-                l_run += p;
+                l_chunk += p;
                 if (col < HG) pbuf[wave][16 * gi + 4 * quad + r][col] = p;
             }
+        l_run += l_chunk;
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();  // the wave's probabilities are in LDS (its accesses stay in order)
+        // Above 128 dims a wave's lane takes every key of the wave: summed by chunk, then over the chunks.
+        constexpr bool BY_CHUNK = D > 128;
+        float part[BY_CHUNK ? HG : 1][VEC] = {};
 #pragma unroll
         for (int j = 0; j < NV; ++j) {
             float p[HG];
@@ -359,9 +386,17 @@ __global__ __launch_bounds__(kThreads) void decode_group_kernel(DecodeArgs a) {
             for (int i = 0; i < VEC; ++i) {
                 const float x = to_f32<T>(vx[j][i]);
 #pragma unroll
-                for (int h = 0; h < HG; ++h) acc[h][i] = fmaf(p[h], x, acc[h][i]);
+                for (int h = 0; h < HG; ++h) {
+                    if constexpr (BY_CHUNK) part[h][i] = fmaf(p[h], x, part[h][i]);
+                    else acc[h][i] = fmaf(p[h], x, acc[h][i]);
+                }
             }
         }
+        if constexpr (BY_CHUNK)
+#pragma unroll
+            for (int h = 0; h < HG; ++h)
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) acc[h][i] += part[h][i];
         __builtin_amdgcn_wave_barrier();
     }
 
