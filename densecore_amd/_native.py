@@ -65,9 +65,9 @@ def _mask_arg(mask, dims, dev):
     return mask, (mask.stride(0), mask.stride(1), mask.stride(2))
 
 
-# DC_FLAG_CONSISTENT_SCORES on every call when set (include/dc_attn.h): the float32 kernels at
-# head dims 65-128 form their scores in one order of products, forward and backward, so that exp(score - lse)
-# normalizes exactly as the forward's did (slower); see consistent_scores().
+# DC_FLAG_CONSISTENT_SCORES on every call when set (include/dc_attn.h): the float32 backward at
+# head dims 65-128 forms its scores in the forward's order of products, so that exp(score - lse)
+# normalizes exactly as the forward's did; the forward does not depend on it; see consistent_scores().
 CONSISTENT_SCORES = False
 
 

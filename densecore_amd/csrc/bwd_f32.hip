@@ -65,7 +65,7 @@ struct alignas(16) BwdSmem {
 
 // Head dim 128 (65 to 128, zero-padded) has two float32 tiles: 8 waves of 16 keys (key_tile16), and 4
 // waves of 32 keys (key_tile) where a caller asks for the forward's score order
-// (AttnShape::consistent).  Waves per SIMD: two and one (one workgroup per CU either way).
+// (AttnShape::consistent; below 128 that is the order of its split products).  Waves per SIMD: two and one (one workgroup per CU either way).
 constexpr int layout_threads(bool k16) { return k16 ? 2 * kThreads : kThreads; }
 constexpr int bwd_waves_per_eu(bool k16) { return k16 ? 2 : 1; }
 
@@ -263,6 +263,41 @@ DEVI int opaque_index(int tid) {
     return tid;
 }
 
+// key_tile's S at head dims whose forward runs on split products (65 to 127, fwd_x3.hip): the same
+// six products in the same order, every small one before the h h ones, so that the scores are the
+// forward's bits.  Q and K are split as they are read (they are in LDS for the other products as
+// float32); a product that is not finite (x3.hpp) is formed again in float32.
+template <int D>
+DEVI void split_scores(const BwdSmem<D> &sm, f32x16 &acc, int wave, int lane) {
+    const int lr = lane & 31, g = lane >> 5;
+    auto q_at = [&](int st) {
+        const f32x4 x[2] = {*reinterpret_cast<const f32x4 *>(&sm.q[lr][16 * st + 8 * g]),
+                            *reinterpret_cast<const f32x4 *>(&sm.q[lr][16 * st + 8 * g + 4])};
+        return split_chunk(x);
+    };
+    auto k_at = [&](int st) {
+        float x[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = sm.kt[16 * st + 8 * g + j][wave * 32 + lr];
+        return split3(x, 0);
+    };
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) {
+        acc = mfma_x3_small_ba(q_at(st), k_at(st), acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int st = 0; st < D / 16; ++st) {
+        acc = mfma_bf16(q_at(st).h, k_at(st).h, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (__any(not_finite(acc) != 0.f)) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+        for (int d = 0; d < D / 2; ++d) acc = mfma_f32(sm.q[lr][g * (D / 2) + d], sm.kt[g * (D / 2) + d][wave * 32 + lr], acc);
+    }
+}
+
 // Steps [i0, i1) of key tile kt of (batch, kv head) bhk, by one workgroup.  The workgroup's dK
 // (times scale) and dV for the tile's keys go to kdst / vdst (the tile's first key row, row
 // stride E): the outputs when these are all of the tile's steps, or the partial slot of the
@@ -387,14 +422,15 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
         f32x16 sacc, pacc;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sacc[r] = 0.f, pacc[r] = 0.f;
+        const bool split = !VEC && s.E < D;  // the forward's products at this head dim
+        if (split) split_scores<D>(sm, sacc, wave, lane);
 #pragma unroll
         for (int t4 = 0; t4 < DH; t4 += 4) {
             const f32x4 qq = *reinterpret_cast<const f32x4 *>(&sm.q[lr][g * DH + t4]);
             const f32x4 oo = *reinterpret_cast<const f32x4 *>(&sm.dout[lr][g * DH + t4]);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
-                const float kk = sm.kt[g * DH + t4 + u][wave * 32 + lr];
-                sacc = mfma_f32(qq[u], kk, sacc);
+                if (!split) sacc = mfma_f32(qq[u], sm.kt[g * DH + t4 + u][wave * 32 + lr], sacc);
                 pacc = mfma_f32(oo[u], vreg[t4 + u], pacc);
             }
             if (t4 % 8 == 4) __builtin_amdgcn_sched_barrier(0);  // bound the hoisted LDS reads

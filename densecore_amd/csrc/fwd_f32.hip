@@ -515,13 +515,11 @@ hipError_t launch_f32(const FwdArgs &args, hipStream_t st) {
 }
 
 // Which kernel a shape takes: up to head dim 127 the split products of fwd_x3.hip (one and a half
-// to three times as fast: causal B2 H12 L4096 D64 439 -> 273 us, B4 H8 L1001 D80 185 -> 68); float32
-// MFMAs at 128, and from 65 up where the caller asks for scores the backward repeats exactly
-// (DC_FLAG_CONSISTENT_SCORES), because the backward of those head dims forms its scores with them.
-// (At 128 the split kernel would take causal B2 H16 L2048 from 357 to 193 us, at half the error; but
-// scores near 100 are held to the reference's own rounding within 2e-5, which it there meets less
-// closely by being nearer the exact result: the reference is off by 2.6e-5.)
-bool split_products(const AttnShape &s) { return s.E <= 64 || (s.E < kD && !s.consistent); }
+// to three times as fast: causal B2 H12 L4096 D64 439 -> 273 us, B4 H8 L1001 D80 185 -> 68), float32
+// MFMAs at 128.  (At 128 the split kernel would take causal B2 H16 L2048 from 357 to 193 us, at half
+// the error; but scores near 100 are held to the reference's own rounding within 2e-5, which it there
+// meets less closely by being nearer the exact result: the reference is off by 2.6e-5.)
+bool split_products(const AttnShape &s) { return s.E < kD; }
 
 }  // namespace
 

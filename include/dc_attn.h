@@ -64,14 +64,15 @@ typedef struct {
     int64_t mask_stride_b, mask_stride_h, mask_stride_l; /* elements; used when mask != NULL */
 } dc_attn_desc;
 
-/* dc_attn_desc.flags.  DC_FLAG_CONSISTENT_SCORES (float32, head dims 65-128): form the
- * backward's scores q.k in the forward's order of products (v_mfma_f32_32x32x2_f32 with the forward's
- * pairing of dims, 32 keys per wave; below 128 the forward then runs on that instruction too, where it
- * otherwise splits every operand exactly into three bf16 parts), so that exp(score - lse) normalizes exactly as the forward's did.
+/* dc_attn_desc.flags.  DC_FLAG_CONSISTENT_SCORES (float32 backward, head dims 65-128): form the
+ * scores q.k in the forward's order of products (at 128 v_mfma_f32_32x32x2_f32 with the forward's
+ * pairing of dims, below it the forward's six bf16 products of operands split exactly in three; 32
+ * keys per wave), so that exp(score - lse) normalizes exactly as the forward's did.  The forward
+ * and its workspace do not depend on it, so it may be set on the backward alone.
  * Without it these head dims take an 8-wave tile of 16 keys on 16x16x4 products (about 20% faster
- * on few-heads shapes), whose scores round in another order: at ordinary scores the results are the
- * same to the float32 bar, at scores near 100 the gradients' error against exact arithmetic grows
- * to a few times the reference's.  No effect elsewhere (head dims up to 64 always use the
+ * on few-heads shapes at 128), whose scores round in another order: at ordinary scores the results
+ * are the same to the float32 bar, at scores near 100 the gradients' error against exact arithmetic
+ * grows to a few times the reference's.  No effect elsewhere (head dims up to 64 always use the
  * forward's order).  Other bits are reserved and must be 0. */
 #define DC_FLAG_CONSISTENT_SCORES 1
 
