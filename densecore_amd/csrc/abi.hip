@@ -154,11 +154,11 @@ size_t fwd_ws(const dc::AttnShape &s, bool bf16) {
 
 // The backward's workspace: dsum (B*H*L floats), then for float32 the deterministic partials
 // (each key tile's dQ slot and the stream-K cut tiles' dK / dV slots; without them dQ is
-// accumulated in its output with atomics), for bf16 the scaled fp16 copies of q, k, v, dout with
+// accumulated in its output with atomics) and a byte per query row (BwdArgs::tame), for bf16 the scaled fp16 copies of q, k, v, dout with
 // their per-slab scratch, then the float32 partials of split grids (small grids on the current
 // device; none otherwise).
 struct BwdLayout {
-    size_t dsum, part, q16, k16, v16, do16, partial, exps, copies_end, split, total;
+    size_t dsum, part, tame, q16, k16, v16, do16, partial, exps, copies_end, split, total;
 };
 BwdLayout bwd_layout(const dc::AttnShape &s, bool bf16) {
     BwdLayout l{};
@@ -175,7 +175,10 @@ BwdLayout bwd_layout(const dc::AttnShape &s, bool bf16) {
         l.total = at;
         return l;
     }
-    if (!bf16) take(dc::bwd_f32_part_bytes(s));
+    if (!bf16) {
+        take(dc::bwd_f32_part_bytes(s));
+        l.tame = take(dc::bwd_f32_tame_bytes(s));
+    }
     if (bf16) {
         const size_t nq = (size_t)s.B * s.H * s.L * s.E, nk = (size_t)s.B * s.Hkv * s.S * s.E;
         const int64_t qslab = (int64_t)s.repeat * s.L * s.E, kslab = (int64_t)s.S * s.E;
@@ -223,18 +226,19 @@ dc::BwdArgs bwd_piece(const dc::BwdArgs &a, int b0, int nb, int hk0, int nh) {
     c.dq_acc = static_cast<float *>(c.dq);
     c.lse = a.lse + qrow * s.L;
     c.dsum = a.dsum + qrow * s.L;
+    c.tame = a.tame ? a.tame + qrow * s.L : nullptr;
     if (s.mask) c.s.mask = s.mask + (int64_t)b0 * s.msb + (int64_t)h0 * s.msh;
     c.s.vec = s.vec && aligned16(c.dout) && aligned16(c.q) && aligned16(c.out) && aligned16(c.k) &&
               aligned16(c.v) && aligned16(c.dq) && aligned16(c.dk) && aligned16(c.dv);
     return c;
 }
 
-// The float32 backward when `avail` bytes of partials (after dsum) are less than the whole
-// problem needs for a result identical from run to run: pieces of whole batches, or of one
-// batch's kv heads, each small enough for its partials to fit, run one after another on the
-// same stream (each piece is a full backward, so the sums keep their fixed order); if not even
-// one kv head fits, the whole problem runs once with float atomics.
-dc_status bwd_f32_chunked(const dc::BwdArgs &a, size_t avail, hipStream_t st) {
+// The pieces of a float32 backward whose partials fit `avail` bytes: nb whole batches each, or
+// (nb == 0) nh kv heads of one batch; both 0 when not even one kv head's partials fit.
+struct Pieces {
+    int nb, nh;
+};
+Pieces bwd_f32_pieces(const dc::BwdArgs &a, size_t avail) {
     const dc::AttnShape &s = a.s;
     auto fits = [&](int nb, int nh) { return dc::bwd_f32_part_bytes(bwd_piece(a, 0, nb, 0, nh).s) <= avail; };
     // The largest piece that fits, stepping down from an estimate (the dQ slots grow linearly with
@@ -246,9 +250,32 @@ dc_status bwd_f32_chunked(const dc::BwdArgs &a, size_t avail, hipStream_t st) {
     };
     const int nb = avail > 0 && s.B > 1 ? largest(s.B, [&](int k) { return fits(k, 0); }) : 0;
     const int nh = avail == 0 || nb >= 1 ? 0 : largest(s.Hkv, [&](int k) { return fits(0, k); });
+    return {std::max(nb, 0), std::max(nh, 0)};
+}
+
+// The float32 backward when the bytes after dsum are fewer than the whole problem's partials, which
+// make its result identical from run to run: pieces of whole batches, or of one batch's kv heads,
+// each small enough for its partials to fit, run one after another on the same stream (each piece
+// is a full backward, so the sums keep their fixed order); if not even one kv head fits, the whole
+// problem runs once with float atomics.  BwdArgs::tame takes the end of the workspace where pieces
+// still fit beside it.
+dc_status bwd_f32_chunked(const dc::BwdArgs &args, size_t avail, hipStream_t st) {
+    dc::BwdArgs a = args;
+    const dc::AttnShape &s = a.s;
+    auto [nb, nh] = bwd_f32_pieces(a, avail);
+    const size_t tame = dc::bwd_f32_tame_bytes(s);
+    if (dc::bwd_f32_skips(s) && avail > tame) {
+        const size_t less = (avail - tame) / 256 * 256;
+        const Pieces beside = bwd_f32_pieces(a, less);
+        if (beside.nb >= 1 || beside.nh >= 1) {
+            nb = beside.nb, nh = beside.nh;
+            a.part_bytes = less;
+            a.tame = reinterpret_cast<uint8_t *>(a.dq_part) + less;
+        }
+    }
     dc::BwdArgs whole = a;
     if (nb < 1 && nh < 1) {  // float atomics over the whole problem
-        whole.dq_part = nullptr, whole.part_bytes = 0;
+        whole.dq_part = nullptr, whole.part_bytes = 0, whole.tame = nullptr;
         return launched(dc::launch_bwd_f32(whole, st));
     }
     int pieces = 0;
@@ -450,6 +477,7 @@ dc_status dc_sdpa_bwd(const dc_attn_desc *d, const void *grad_out, const void *q
     if (!bf16 && s.E <= dc::kFlashMaxHeadDim && workspace_bytes > l.part) {
         a.dq_part = reinterpret_cast<float *>(ws + l.part);
         a.part_bytes = workspace_bytes - l.part;
+        if (dc::bwd_f32_skips(s) && workspace_bytes >= l.total) a.tame = reinterpret_cast<uint8_t *>(ws + l.tame);
     }
     // bf16: the fp16 products when the workspace holds the copies (else the bf16 hi + lo pairs).
     if (bf16 && workspace_bytes >= l.copies_end) {
@@ -462,7 +490,7 @@ dc_status dc_sdpa_bwd(const dc_attn_desc *d, const void *grad_out, const void *q
         }
     }
     hipStream_t strm = static_cast<hipStream_t>(stream);
-    if (!bf16 && s.E <= dc::kFlashMaxHeadDim && workspace_bytes < l.total) {
+    if (!bf16 && s.E <= dc::kFlashMaxHeadDim && workspace_bytes - l.part < dc::bwd_f32_part_bytes(s)) {
         // The whole problem's deterministic partials do not fit: run it in pieces whose do.
         st = bwd_f32_chunked(a, workspace_bytes - l.part, strm);
         if (st != DC_OK) return st;

@@ -636,7 +636,7 @@ struct alignas(16) BwdSmemX3 {
     X3Tile<32, 32> ds[kWaves];       // dS: rows are keys, columns the step's queries
     float part[kWaves][kBM][D + 4];  // a wave's share of dQ
     float lse[2][kBM], dsum[2][kBM];
-    int open[kWaves];                // row masks: the wave's keys have one that is not -inf
+    int seen[2 * kWaves];            // row masks: bit 0, the wave's keys have one that is not -inf; bit 1, tame
 };
 
 // MASK: 0 none, 1 a value per (query, key), 2 the same for every query (key padding).
@@ -672,18 +672,36 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         if (dq_atomic) return a.dq_acc + ((int64_t)p.bh * s.L + p.m0) * s.E;
         return a.dq_part + (slot0 + (int64_t)p.bh * (s.L - rf) + (p.m0 - rf)) * s.E;
     };
-    // Padding: a wave none of whose keys is visible to any query does no work (masks that differ
-    // between heads are not looked at).
+    // Padding: a wave none of whose keys is visible to any query does no work where that is exact
+    // (masks that differ between heads are not looked at).  The visit would add P = exp(-inf - lse) = 0
+    // times dO to dV and 0 times (dO V - dsum), Q and K to the others: zeros, unless a score, dO V or an
+    // operand is not finite (the reference's 0 * NaN).  So the rows must be tame (bwd_pre_block) and the
+    // masked keys' K and V too; otherwise every key of the tile is visited.
     int open = 15;
-    if (MASK == 2 && s.msh == 0) {
-        __syncthreads();  // a previous tile's last readers of sm.open are done
-        if (group_a) {
-            const bool any = __any(key < s.S && mbase[min(key, s.S - 1)] != -INFINITY);
-            if (lane == 0) sm.open[wave] = any;
+    auto look = [&](bool &any, bool &tame) {  // this wave's part
+        any = __any(key < s.S && mbase[min(key, s.S - 1)] != -INFINITY);
+        tame = true;
+        for (int j = tid; j < (i1 - i0) * kBM; j += kX3Threads) {
+            const int i = i0 + j / kBM, qq = m_begin + (i % per_head) * kBM + j % kBM;
+            if (qq < s.L) tame &= a.tame[(int64_t)(b * s.H + hk * s.repeat + i / per_head) * s.L + qq] != 0;
         }
-        __syncthreads();
-        open = __builtin_amdgcn_readfirstlane(sm.open[0] | sm.open[1] << 1 | sm.open[2] << 2 | sm.open[3] << 3);
-    }
+        if (!any && kw0 < s.S) {  // the wave's 32 rows of K (group A) or V (group B)
+            const float *rows = static_cast<const float *>(group_a ? a.k : a.v) + ((int64_t)bhk * s.S + kw0) * s.E;
+            const int count = min(32, s.S - kw0) * s.E;
+            if constexpr (VEC) {
+#pragma unroll 8
+                for (int j = 4 * lane; j < count; j += 256) {
+                    const f32x4 x = *reinterpret_cast<const f32x4 *>(rows + j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) tame &= fabsf(x[e]) <= kTame;
+                }
+            } else {
+#pragma unroll 8
+                for (int j = lane; j < count; j += 64) tame &= fabsf(rows[j]) <= kTame;
+            }
+        }
+        tame = __all(tame);
+    };
     // Wave w works in a step if some query of the step sees one of its keys.
     auto live_at = [&](int w, int m0) {
         return ((open >> w) & 1) && n0 + 32 * w < s.S && (!CAUSAL || m0 + kBM - 1 >= n0 + 32 * w);
@@ -719,16 +737,7 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             }
     };
 
-    if (i0 < i1 && open == 0) {  // nothing visible: the tile's dQ shares are zero
-        if (!dq_atomic) {
-            Pos p = first;
-            for (int i = i0; i < i1; ++i, p = next_pos(p)) {
-                float *dst = dq_dst(p);
-                const int count = min(kBM, s.L - p.m0) * s.E;
-                for (int j = tid; j < count; j += kX3Threads) dst[j] = 0.f;
-            }
-        }
-    } else if (i0 < i1) {
+    if (i0 < i1) {
         // Group A stages dO (with lse and dsum), group B Q: a step at a time, in registers until the
         // buffer it goes to is free.
         X3Stage<kBM, D, kThreads, VEC> stage;
@@ -753,21 +762,42 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         // tile w): K as A's row operand and B's transposed one, then V as B's row operand.  The first
         // steps' Q and dO are on their way meanwhile.
         X3 kv[KSTEP], kT[NDT][2];
-        {
-            static_assert(kWaves * sizeof(X3Tile<kBM, D>) <= sizeof(sm.ds) + sizeof(sm.part), "the rows fit");
-            X3Tile<kBM, D> &wt = reinterpret_cast<X3Tile<kBM, D> *>(&sm.ds[0])[wave];
-            X3Stage<kBM, D, 64, VEC> rows;
-            rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, lane);
-            load_step();
-            __syncthreads();  // a previous tile's last readers of these areas are done
-            if (group_a) {
-                rows.store(wt, lane);
-                store_do(0);
-            } else {
-                stage.store(sm.q[0], gtid);
+        static_assert(kWaves * sizeof(X3Tile<kBM, D>) <= sizeof(sm.ds) + sizeof(sm.part), "the rows fit");
+        X3Tile<kBM, D> &wt = reinterpret_cast<X3Tile<kBM, D> *>(&sm.ds[0])[wave];
+        X3Stage<kBM, D, 64, VEC> rows;
+        rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, lane);
+        load_step();
+        bool any = true, tame = true;
+        if (MASK == 2 && a.tame) look(any, tame);
+        __syncthreads();  // a previous tile's last readers of these areas are done
+        if (MASK == 2 && lane == 0) sm.seen[wave8] = (any ? 1 : 0) | (tame ? 2 : 0);
+        if (group_a) {
+            rows.store(wt, lane);
+            store_do(0);
+        } else {
+            stage.store(sm.q[0], gtid);
+        }
+        if (i0 + 1 < i1) load_step();
+        __syncthreads();
+        if (MASK == 2 && a.tame) {
+            int all = 2, seen = 0;
+#pragma unroll
+            for (int w = 0; w < 2 * kWaves; ++w) {
+                const int x = sm.seen[w];
+                all &= x, seen |= (x & 1) << (w & 3);
             }
-            if (i0 + 1 < i1) load_step();
-            __syncthreads();
+            open = __builtin_amdgcn_readfirstlane(all ? seen : 15);
+        }
+        if (open == 0) {  // nothing visible: the tile's dQ shares are zero
+            if (!dq_atomic) {
+                Pos p = first;
+                for (int i = i0; i < i1; ++i, p = next_pos(p)) {
+                    float *dst = dq_dst(p);
+                    const int count = min(kBM, s.L - p.m0) * s.E;
+                    for (int j = tid; j < count; j += kX3Threads) dst[j] = 0.f;
+                }
+            }
+        } else {
             if (group_a) {
 #pragma unroll
                 for (int st = 0; st < KSTEP; ++st) kv[st] = row_frag_x3(wt, rowb, 0, st);
@@ -788,205 +818,205 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
                     if (i0 + 2 < i1) load_step();
                 }
             }
-        }
-        __syncthreads();  // Q of the first two steps, dO of the first
+            __syncthreads();  // Q of the first two steps, dO of the first
 
-        Pos pos = first, prev{-1, 0};
-        bool live = live_at(wave, pos.m0);
-        if (group_a) {
-            float mrow = 0.f;
-            int mrow_bh = -1;
-            float mfull[MASK == 1 ? 16 : 1];
-            auto full_mask = [&](Pos p) {  // the mask of the step at p
-                if constexpr (MASK == 1) {
+            Pos pos = first, prev{-1, 0};
+            bool live = live_at(wave, pos.m0);
+            if (group_a) {
+                float mrow = 0.f;
+                int mrow_bh = -1;
+                float mfull[MASK == 1 ? 16 : 1];
+                auto full_mask = [&](Pos p) {  // the mask of the step at p
+                    if constexpr (MASK == 1) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int qq = p.m0 + acc_row(r, g);
-                        mfull[r] = (qq < s.L && key < s.S) ? mbase[(int64_t)(p.bh - b * s.H) * s.msh + (int64_t)qq * s.msl + key] : 0.f;
+                        for (int r = 0; r < 16; ++r) {
+                            const int qq = p.m0 + acc_row(r, g);
+                            mfull[r] = (qq < s.L && key < s.S) ? mbase[(int64_t)(p.bh - b * s.H) * s.msh + (int64_t)qq * s.msl + key] : 0.f;
+                        }
                     }
-                }
-            };
-            f32x16 sacc;
-            X3 p3[2];
-            // S = Q K^T (queries are rows, the wave's keys columns), in k-step groups; and dV += P^T dO,
-            // in groups of 32 dims by 16 queries.
-            auto score_group = [&](int st, const X3 &q) {
-                if (st == 0) {
+                };
+                f32x16 sacc;
+                X3 p3[2];
+                // S = Q K^T (queries are rows, the wave's keys columns), in k-step groups; and dV += P^T dO,
+                // in groups of 32 dims by 16 queries.
+                auto score_group = [&](int st, const X3 &q) {
+                    if (st == 0) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
-                }
-                sacc = mfma_x3_small_ba(q, kv[st], sacc);
-            };
-            auto score_rest = [&](int buf) {
+                        for (int r = 0; r < 16; ++r) sacc[r] = 0.f;
+                    }
+                    sacc = mfma_x3_small_ba(q, kv[st], sacc);
+                };
+                auto score_rest = [&](int buf) {
 #pragma unroll
-                for (int st = 0; st < KSTEP; ++st)
-                    sacc = mfma_bf16(row_frag<kBM, D>(sm.q[buf].p[0], rowb, 0, st), kv[st].h, sacc);
-            };
-            auto value_group = [&](int gi, const X3 &o) { acc[gi % NDT] = mfma_x3(o, p3[gi / NDT], acc[gi % NDT]); };
-            auto scores = [&](int buf) {
-                pipelined<KSTEP>([&](int st) { return row_frag_x3(sm.q[buf], rowb, 0, st); }, score_group);
-                score_rest(buf);
-            };
-            if (live) {
-                full_mask(pos);
-                scores(0);
-            }
-            int qb = 0;  // buffer of Q(i)
-            for (int i = i0; i < i1; ++i) {
-                const Pos npos = next_pos(pos);
-                const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
-                const int ob = (i - i0) & 1;
-                qb = qb == 2 ? 0 : qb + 1;  // of Q(i + 1)
+                    for (int st = 0; st < KSTEP; ++st)
+                        sacc = mfma_bf16(row_frag<kBM, D>(sm.q[buf].p[0], rowb, 0, st), kv[st].h, sacc);
+                };
+                auto value_group = [&](int gi, const X3 &o) { acc[gi % NDT] = mfma_x3(o, p3[gi / NDT], acc[gi % NDT]); };
+                auto scores = [&](int buf) {
+                    pipelined<KSTEP>([&](int st) { return row_frag_x3(sm.q[buf], rowb, 0, st); }, score_group);
+                    score_rest(buf);
+                };
                 if (live) {
-                    if (MASK == 2 && pos.bh != mrow_bh) {
-                        mrow = key < s.S ? mbase[(int64_t)(pos.bh - b * s.H) * s.msh + key] : 0.f;
-                        mrow_bh = pos.bh;
+                    full_mask(pos);
+                    scores(0);
+                }
+                int qb = 0;  // buffer of Q(i)
+                for (int i = i0; i < i1; ++i) {
+                    const Pos npos = next_pos(pos);
+                    const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
+                    const int ob = (i - i0) & 1;
+                    qb = qb == 2 ? 0 : qb + 1;  // of Q(i + 1)
+                    if (live) {
+                        if (MASK == 2 && pos.bh != mrow_bh) {
+                            mrow = key < s.S ? mbase[(int64_t)(pos.bh - b * s.H) * s.msh + key] : 0.f;
+                            mrow_bh = pos.bh;
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const f32x4 l4 = *reinterpret_cast<const f32x4 *>(&sm.lse[ob][8 * j + 4 * g]);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                // scale * q.k (+ mask) - lse in natural-log units, as the reference forms
+                                // it, then one conversion to base 2 for v_exp_f32.
+                                const int r = 4 * j + e;
+                                float x = sacc[r] * s.scale;
+                                if (MASK == 1) x += mfull[MASK == 1 ? r : 0];
+                                if (MASK == 2) x += mrow;
+                                sacc[r] = exp2_fast((x - l4[e]) * kLog2e);
+                            }
+                        }
+                        // Keys past the end or (causal) past a query only occur when the wave's keys reach
+                        // the end of the sequence or cross the diagonal of this query tile.
+                        if (kw0 + 31 >= s.S || (CAUSAL && kw0 + 31 > pos.m0)) {
+                            asm volatile("" ::: "memory");  // keeps the branch: not if-converted into selects
+#pragma unroll
+                            for (int r = 0; r < 16; ++r)
+                                if (key >= s.S || (CAUSAL && key > pos.m0 + acc_row(r, g))) sacc[r] = 0.f;
+                        }
+#pragma unroll
+                        for (int r = 0; r < 16; ++r) sm.p[wave][r][lane] = sacc[r];
+                        p3[0] = split3(sacc, 0);
+                        p3[1] = split3(sacc, 8);
                     }
+                    if (i + 1 < i1) {
+                        store_do(ob ^ 1);
+                        if (i + 2 < i1) load_step();
+                    }
+                    __syncthreads();
+                    if (nlive) full_mask(npos);
+                    auto read_do = [&](int gi) { return tr_frag_x3(sm.o[ob], trb, 16 * (gi / NDT), gi % NDT); };
+                    if (live && nlive) {
+                        pipelined<2 * NDT + KSTEP>(
+                            [&](int k) { return k < 2 * NDT ? read_do(k) : row_frag_x3(sm.q[qb], rowb, 0, k - 2 * NDT); },
+                            [&](int k, const X3 &f) {
+                                if (k < 2 * NDT) value_group(k, f);
+                                else score_group(k - 2 * NDT, f);
+                            });
+                        score_rest(qb);
+                    } else {
+                        if (live) pipelined<2 * NDT>(read_do, value_group);
+                        if (nlive) scores(qb);
+                    }
+                    if (prev.bh >= 0) reduce_dq(prev);
+                    live = nlive;
+                    prev = pos, pos = npos;
+                    __syncthreads();
+                }
+                __syncthreads();
+            } else {
+                const uint32_t dstrb = tr_lanebase<32, 32>(lane);
+                f32x16 pacc;
+                X3 d3[2];
+                auto dq_share = [&]() {  // of the step whose dS is in the wave's tile
+                    const X3 dsT[2] = {tr_frag_x3(sm.ds[wave], dstrb, 0, 0), tr_frag_x3(sm.ds[wave], dstrb, 16, 0)};
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const f32x4 l4 = *reinterpret_cast<const f32x4 *>(&sm.lse[ob][8 * j + 4 * g]);
+                    for (int dt = 0; dt < NDT; ++dt) {
+                        f32x16 dq;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            // scale * q.k (+ mask) - lse in natural-log units, as the reference forms
-                            // it, then one conversion to base 2 for v_exp_f32.
-                            const int r = 4 * j + e;
-                            float x = sacc[r] * s.scale;
-                            if (MASK == 1) x += mfull[MASK == 1 ? r : 0];
-                            if (MASK == 2) x += mrow;
-                            sacc[r] = exp2_fast((x - l4[e]) * kLog2e);
+                        for (int r = 0; r < 16; ++r) dq[r] = 0.f;
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) dq = mfma_x3(kT[dt][u], dsT[u], dq);
+#pragma unroll
+                        for (int r = 0; r < 16; r += 4)
+                            *reinterpret_cast<f32x4 *>(&sm.part[wave][lr][32 * dt + acc_row(r, g)]) =
+                                f32x4{dq[r], dq[r + 1], dq[r + 2], dq[r + 3]};
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                };
+                auto key_group = [&](int gi, const X3 &q) { acc[gi % NDT] = mfma_x3(q, d3[gi / NDT], acc[gi % NDT]); };
+                auto prob_group = [&](int st, const X3 &o) { pacc = mfma_x3(o, kv[st], pacc); };
+                int pb = 2;  // buffer of Q(i - 1)
+                bool plive = false;
+                for (int i = i0; i < i1; ++i) {
+                    const Pos npos = next_pos(pos);
+                    const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
+                    const int ob = (i - i0) & 1;
+                    // dK += dS^T Q of the step before, and dP = dO V^T.
+                    auto read_q = [&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); };
+                    auto read_do = [&](int st) { return row_frag_x3(sm.o[ob], rowb, 0, st); };
+                    if (plive) dq_share();
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) pacc[r] = 0.f;
+                    if (plive && live) {
+                        pipelined<2 * NDT + KSTEP>([&](int k) { return k < 2 * NDT ? read_q(k) : read_do(k - 2 * NDT); },
+                                                   [&](int k, const X3 &f) {
+                                                       if (k < 2 * NDT) key_group(k, f);
+                                                       else prob_group(k - 2 * NDT, f);
+                                                   });
+                    } else {
+                        if (plive) pipelined<2 * NDT>(read_q, key_group);
+                        if (live) pipelined<KSTEP>(read_do, prob_group);
+                    }
+                    __syncthreads();
+                    if (live) {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&sm.dsum[ob][8 * j + 4 * g]);
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) {
+                                const int r = 4 * j + e;
+                                pacc[r] = sm.p[wave][r][lane] * (pacc[r] - d4[e]);
+                            }
+                        }
+                        // Into the dS tile: rows are keys, columns queries (registers 8u .. 8u + 7 hold
+                        // queries 16u + 4g + 0..3 and 16u + 8 + 4g + 0..3).
+#pragma unroll
+                        for (int u = 0; u < 2; ++u) {
+                            d3[u] = split3(pacc, 8 * u);
+                            const bf16x8 parts[3] = {d3[u].h, d3[u].m, d3[u].l};
+#pragma unroll
+                            for (int pl = 0; pl < 3; ++pl) {
+                                const u32x4 w = __builtin_bit_cast(u32x4, parts[pl]);
+                                uint32_t *row = reinterpret_cast<uint32_t *>(&sm.ds[wave].p[pl][2 * u * CMTile<32, 32>::P + lr]) + 2 * g;
+                                *reinterpret_cast<uint64_t *>(row) = (uint64_t)w[0] | ((uint64_t)w[1] << 32);
+                                *reinterpret_cast<uint64_t *>(row + CMTile<32, 32>::P * 4) = (uint64_t)w[2] | ((uint64_t)w[3] << 32);
+                            }
                         }
                     }
-                    // Keys past the end or (causal) past a query only occur when the wave's keys reach
-                    // the end of the sequence or cross the diagonal of this query tile.
-                    if (kw0 + 31 >= s.S || (CAUSAL && kw0 + 31 > pos.m0)) {
-                        asm volatile("" ::: "memory");  // keeps the branch: not if-converted into selects
-#pragma unroll
-                        for (int r = 0; r < 16; ++r)
-                            if (key >= s.S || (CAUSAL && key > pos.m0 + acc_row(r, g))) sacc[r] = 0.f;
+                    if (prev.bh >= 0) reduce_dq(prev);
+                    if (i + 2 < i1) {
+                        stage.store(sm.q[pb], gtid);  // Q(i + 2) where Q(i - 1) was
+                        if (i + 3 < i1) load_step();
                     }
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) sm.p[wave][r][lane] = sacc[r];
-                    p3[0] = split3(sacc, 0);
-                    p3[1] = split3(sacc, 8);
+                    pb = pb == 2 ? 0 : pb + 1;
+                    plive = live, live = nlive;
+                    prev = pos, pos = npos;
+                    __syncthreads();
                 }
-                if (i + 1 < i1) {
-                    store_do(ob ^ 1);
-                    if (i + 2 < i1) load_step();
+                if (plive) {
+                    dq_share();
+                    pipelined<2 * NDT>([&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); }, key_group);
                 }
-                __syncthreads();
-                if (nlive) full_mask(npos);
-                auto read_do = [&](int gi) { return tr_frag_x3(sm.o[ob], trb, 16 * (gi / NDT), gi % NDT); };
-                if (live && nlive) {
-                    pipelined<2 * NDT + KSTEP>(
-                        [&](int k) { return k < 2 * NDT ? read_do(k) : row_frag_x3(sm.q[qb], rowb, 0, k - 2 * NDT); },
-                        [&](int k, const X3 &f) {
-                            if (k < 2 * NDT) value_group(k, f);
-                            else score_group(k - 2 * NDT, f);
-                        });
-                    score_rest(qb);
-                } else {
-                    if (live) pipelined<2 * NDT>(read_do, value_group);
-                    if (nlive) scores(qb);
-                }
-                if (prev.bh >= 0) reduce_dq(prev);
-                live = nlive;
-                prev = pos, pos = npos;
                 __syncthreads();
             }
-            __syncthreads();
-        } else {
-            const uint32_t dstrb = tr_lanebase<32, 32>(lane);
-            f32x16 pacc;
-            X3 d3[2];
-            auto dq_share = [&]() {  // of the step whose dS is in the wave's tile
-                const X3 dsT[2] = {tr_frag_x3(sm.ds[wave], dstrb, 0, 0), tr_frag_x3(sm.ds[wave], dstrb, 16, 0)};
-#pragma unroll
-                for (int dt = 0; dt < NDT; ++dt) {
-                    f32x16 dq;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) dq[r] = 0.f;
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) dq = mfma_x3(kT[dt][u], dsT[u], dq);
-#pragma unroll
-                    for (int r = 0; r < 16; r += 4)
-                        *reinterpret_cast<f32x4 *>(&sm.part[wave][lr][32 * dt + acc_row(r, g)]) =
-                            f32x4{dq[r], dq[r + 1], dq[r + 2], dq[r + 3]};
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            };
-            auto key_group = [&](int gi, const X3 &q) { acc[gi % NDT] = mfma_x3(q, d3[gi / NDT], acc[gi % NDT]); };
-            auto prob_group = [&](int st, const X3 &o) { pacc = mfma_x3(o, kv[st], pacc); };
-            int pb = 2;  // buffer of Q(i - 1)
-            bool plive = false;
-            for (int i = i0; i < i1; ++i) {
-                const Pos npos = next_pos(pos);
-                const bool nlive = i + 1 < i1 && live_at(wave, npos.m0);
-                const int ob = (i - i0) & 1;
-                // dK += dS^T Q of the step before, and dP = dO V^T.
-                auto read_q = [&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); };
-                auto read_do = [&](int st) { return row_frag_x3(sm.o[ob], rowb, 0, st); };
-                if (plive) dq_share();
-#pragma unroll
-                for (int r = 0; r < 16; ++r) pacc[r] = 0.f;
-                if (plive && live) {
-                    pipelined<2 * NDT + KSTEP>([&](int k) { return k < 2 * NDT ? read_q(k) : read_do(k - 2 * NDT); },
-                                               [&](int k, const X3 &f) {
-                                                   if (k < 2 * NDT) key_group(k, f);
-                                                   else prob_group(k - 2 * NDT, f);
-                                               });
-                } else {
-                    if (plive) pipelined<2 * NDT>(read_q, key_group);
-                    if (live) pipelined<KSTEP>(read_do, prob_group);
-                }
-                __syncthreads();
-                if (live) {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const f32x4 d4 = *reinterpret_cast<const f32x4 *>(&sm.dsum[ob][8 * j + 4 * g]);
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const int r = 4 * j + e;
-                            pacc[r] = sm.p[wave][r][lane] * (pacc[r] - d4[e]);
-                        }
-                    }
-                    // Into the dS tile: rows are keys, columns queries (registers 8u .. 8u + 7 hold
-                    // queries 16u + 4g + 0..3 and 16u + 8 + 4g + 0..3).
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        d3[u] = split3(pacc, 8 * u);
-                        const bf16x8 parts[3] = {d3[u].h, d3[u].m, d3[u].l};
-#pragma unroll
-                        for (int pl = 0; pl < 3; ++pl) {
-                            const u32x4 w = __builtin_bit_cast(u32x4, parts[pl]);
-                            uint32_t *row = reinterpret_cast<uint32_t *>(&sm.ds[wave].p[pl][2 * u * CMTile<32, 32>::P + lr]) + 2 * g;
-                            *reinterpret_cast<uint64_t *>(row) = (uint64_t)w[0] | ((uint64_t)w[1] << 32);
-                            *reinterpret_cast<uint64_t *>(row + CMTile<32, 32>::P * 4) = (uint64_t)w[2] | ((uint64_t)w[3] << 32);
-                        }
-                    }
-                }
-                if (prev.bh >= 0) reduce_dq(prev);
-                if (i + 2 < i1) {
-                    stage.store(sm.q[pb], gtid);  // Q(i + 2) where Q(i - 1) was
-                    if (i + 3 < i1) load_step();
-                }
-                pb = pb == 2 ? 0 : pb + 1;
-                plive = live, live = nlive;
-                prev = pos, pos = npos;
-                __syncthreads();
-            }
-            if (plive) {
-                dq_share();
-                pipelined<2 * NDT>([&](int gi) { return tr_frag_x3(sm.q[pb], trb, 16 * (gi / NDT), gi % NDT); }, key_group);
-            }
-            __syncthreads();
-        }
-        reduce_dq(prev);
+            reduce_dq(prev);
 
-        // Not finite: the tile's steps again in plain float32 (x3.hpp).
-        float bad = 0.f;
+            // Not finite: the tile's steps again in plain float32 (x3.hpp).
+            float bad = 0.f;
 #pragma unroll
-        for (int dt = 0; dt < NDT; ++dt) bad += not_finite(acc[dt]);
-        if (__syncthreads_or(bad != 0.f)) redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+            for (int dt = 0; dt < NDT; ++dt) bad += not_finite(acc[dt]);
+            if (__syncthreads_or(bad != 0.f)) redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+        }
     }
 
     // dV, or dK times scale, of this lane's key.
@@ -1411,7 +1441,8 @@ DEVI SkTile sk_tile(const AttnShape &s, const StreamK &sk, int bhk, int kt) {
 // that no single workgroup owns (cut, or without steps: nobody writes it).
 __global__ __launch_bounds__(256) void bwd_pre_f32_kernel(BwdArgs a, StreamK sk, int rows_blocks) {
     if ((int)blockIdx.x < rows_blocks) {
-        if (a.dq_part) bwd_pre_block<float, false>(a, blockIdx.x);
+        if (a.tame) bwd_pre_block<float, false, true>(a, blockIdx.x);
+        else if (a.dq_part) bwd_pre_block<float, false>(a, blockIdx.x);
         else bwd_pre_block<float, true>(a, blockIdx.x);
         return;
     }
@@ -1615,7 +1646,7 @@ hipError_t launch_d(const BwdArgs &args, size_t part_bytes, hipStream_t st) {
     if (a.dq_part && dq_bytes + kv_part_bytes(sk, a.s.E) <= part_bytes) {
         a.kv_part = sk.chunks > 0 ? a.dq_part + dq_bytes / sizeof(float) : nullptr;
     } else {
-        a.dq_part = a.kv_part = nullptr;
+        a.dq_part = a.kv_part = nullptr, a.tame = nullptr;
     }
     record_schedule(deterministic, a.dq_part ? 1 : 0);
     const int64_t rows = (int64_t)a.s.B * a.s.H * a.s.L;

@@ -61,6 +61,10 @@ struct BwdArgs {
     // slot, summed in range order.  nullptr: float atomics into dq (and dk / dv of cut tiles).
     float *dq_part, *kv_part;
     size_t part_bytes;  // workspace bytes at dq_part
+    // float32 key padding at head dims up to 64 (when the workspace holds it): whether a row of q and
+    // dout (B, H, L) is small enough that keys masked for every query take nothing from it
+    // (bwd_f32.hip).  nullptr: masked keys are visited like any other.
+    uint8_t *tame;
     // bf16: q, k, v, dout copied to fp16 (f16_stage.hip), each scaled by 2^e per (b, kv head)
     // (q and dout per group of query heads sharing a kv head); exps holds e_q, e_k, e_v, e_do,
     // B*Hkv each.  nullptr: P and dS enter their products as bf16 hi + lo.
@@ -173,6 +177,13 @@ hipError_t launch_bwd_f32(const BwdArgs &a, hipStream_t st);
 // Workspace bytes of the float32 backward's deterministic partials on the current device (dQ
 // slots, then the stream-K cut tiles' dK / dV slots), with or without a mask.
 size_t bwd_f32_part_bytes(const AttnShape &s);
+// Bytes of BwdArgs::tame (0: this shape's kernels do not use it), and whether a call's mask and scale
+// let masked keys be skipped at all.
+inline size_t bwd_f32_tame_bytes(const AttnShape &s) { return s.E <= 64 ? (size_t)s.B * s.H * s.L : 0; }
+constexpr float kTameScale = 256.f;
+inline bool bwd_f32_skips(const AttnShape &s) {
+    return s.mask && s.msl == 0 && s.msh == 0 && s.E <= 64 && s.scale >= -kTameScale && s.scale <= kTameScale;
+}
 hipError_t launch_bwd_bf16(const BwdArgs &a, hipStream_t st);
 // Workspace bytes the bf16 backward uses to split its grids on the current device (0: it does not
 // split this shape).

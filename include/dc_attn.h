@@ -98,7 +98,8 @@ dc_status dc_sdpa_fwd(const dc_attn_desc *d, const void *q, const void *k, const
  * the size returned also covers, for float32, the partials that make the result identical from
  * run to run (each key tile's dQ share, and on few-tile grids the dK / dV shares of key tiles
  * split between workgroups, summed in a fixed order; with less, these shares are added with
- * float atomics and the last bits of dq, dk, dv can vary between runs), for bf16, scaled fp16
+ * float atomics and the last bits of dq, dk, dv can vary between runs) and a byte per query row
+ * (with less, keys that a padding mask hides are visited, to the same result), for bf16, scaled fp16
  * copies of q, k, v and grad_out (with less, P and dS enter their products as bf16 hi + lo
  * pairs) and, for bf16 without a mask on grids that fill at most half of the current device,
  * the float32 partials of its split grids.  The size depends on the device current at the call
