@@ -65,9 +65,13 @@ struct alignas(16) BwdSmem {
 
 // Head dim 128 (65 to 128, zero-padded) has two float32 tiles: 8 waves of 16 keys (key_tile16), and 4
 // waves of 32 keys (key_tile) where a caller asks for the forward's score order
-// (AttnShape::consistent; below 128 that is the order of its split products).  Waves per SIMD: two and one (one workgroup per CU either way).
+// (AttnShape::consistent; below 128 that is the order of its split products): two waves per SIMD and
+// one, one workgroup per CU either way.  Head dims up to 64 take key_tile where the workspace holds no
+// slots: the shares then go out with float atomics, which key_tile_x3's eight waves would issue in
+// longer runs (causal B8 H12 L1024 D64 390 us against 335), and an infinity's split NaN, once added,
+// could not be taken back.  Two workgroups per CU without a mask, one with.
 constexpr int layout_threads(bool k16) { return k16 ? 2 * kThreads : kThreads; }
-constexpr int bwd_waves_per_eu(bool k16) { return k16 ? 2 : 1; }
+constexpr int bwd_waves_per_eu(int D, bool mask, bool k16) { return k16 || (D <= 64 && !mask) ? 2 : 1; }
 
 // Register staging of one step's Q and dO rows (fast path: E == D, 16-byte aligned).
 template <int D, int NT>
@@ -263,32 +267,26 @@ DEVI int opaque_index(int tid) {
     return tid;
 }
 
-// key_tile's S at head dims whose forward runs on split products (65 to 127, fwd_x3.hip): the same
-// six products in the same order, every small one before the h h ones, so that the scores are the
-// forward's bits.  Q and K are split as they are read (they are in LDS for the other products as
-// float32); a product that is not finite (x3.hpp) is formed again in float32.
-template <int D>
-DEVI void split_scores(const BwdSmem<D> &sm, f32x16 &acc, int wave, int lane) {
+// key_tile's S where the forward runs on split products (head dims up to 127, fwd_x3.hip): the same six
+// products in the same order, every small one before the h h ones, so that the scores are the
+// forward's bits.  Q is split as it is read from LDS, K (k(st): dims 16 st + 8 g .. of the lane's key)
+// by the caller; sums that are not finite (x3.hpp) are formed again in float32.
+template <int D, typename F>
+DEVI void split_scores(const BwdSmem<D> &sm, f32x16 &acc, F k, int wave, int lane) {
     const int lr = lane & 31, g = lane >> 5;
-    auto q_at = [&](int st) {
+    auto q = [&](int st) {
         const f32x4 x[2] = {*reinterpret_cast<const f32x4 *>(&sm.q[lr][16 * st + 8 * g]),
                             *reinterpret_cast<const f32x4 *>(&sm.q[lr][16 * st + 8 * g + 4])};
         return split_chunk(x);
     };
-    auto k_at = [&](int st) {
-        float x[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = sm.kt[16 * st + 8 * g + j][wave * 32 + lr];
-        return split3(x, 0);
-    };
 #pragma unroll
     for (int st = 0; st < D / 16; ++st) {
-        acc = mfma_x3_small_ba(q_at(st), k_at(st), acc);
+        acc = mfma_x3_small_ba(q(st), k(st), acc);
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int st = 0; st < D / 16; ++st) {
-        acc = mfma_bf16(q_at(st).h, k_at(st).h, acc);
+        acc = mfma_bf16(q(st).h, k(st).h, acc);
         __builtin_amdgcn_sched_barrier(0);
     }
     if (__any(not_finite(acc) != 0.f)) {
@@ -318,15 +316,26 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
     const float *kb = static_cast<const float *>(a.k) + (int64_t)bhk * s.S * s.E;
     const float *vb = static_cast<const float *>(a.v) + (int64_t)bhk * s.S * s.E;
 
-    // V row of this lane's key: V[key][g*DH + t].  The K row is not held in registers: S reads it from
-    // the workgroup's transposed K tile in LDS (which the dQ product needs anyway), one ds_read_b32
-    // of 32 consecutive keys per half-wave and MFMA.  K and V rows plus the dK / dV accumulators
-    // (4 x 64 floats per lane) would not fit one wave's registers without spills.
+    // V row of this lane's key: V[key][g*DH + t].  Up to 64 dims K is split once and held in registers
+    // too.  At D = 128 it is not: S reads it from the workgroup's transposed K tile in LDS (which the
+    // dQ product needs anyway), one ds_read_b32 of 32 consecutive keys per half-wave and MFMA.  K and V
+    // rows plus the dK / dV accumulators (4 x 64 floats per lane) would not fit one wave's registers
+    // without spills.
+    constexpr bool KREG = D <= 64;
+    X3 k3[KREG ? D / 16 : 1];
     float vreg[DH];
     const int ptid = opaque_index(tid);  // the prologue's own copy (see opaque_index)
     const int pkey = kw0 + (ptid & 31), pg = (ptid & 63) >> 5;
     {
         const float *vr = vb + (int64_t)pkey * s.E;
+        if constexpr (KREG) {
+#pragma unroll
+            for (int st = 0; st < D / 16; ++st) {
+                f32x4 x[2] = {};
+                if (pkey < s.S) load_chunk<VEC>(x, kb + (int64_t)pkey * s.E, 16 * st + 8 * pg, s.E);
+                k3[st] = split_chunk(x);
+            }
+        }
         if (VEC && pkey < s.S) {
 #pragma unroll
             for (int t = 0; t < DH; t += 4) {
@@ -422,8 +431,15 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
         f32x16 sacc, pacc;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sacc[r] = 0.f, pacc[r] = 0.f;
-        const bool split = !VEC && s.E < D;  // the forward's products at this head dim
-        if (split) split_scores<D>(sm, sacc, wave, lane);
+        const bool split = KREG || (!VEC && s.E < D);  // the forward's products at this head dim
+        if (split)
+            split_scores<D>(sm, sacc, [&](int st) {
+                if constexpr (KREG) return k3[st];
+                float x[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = sm.kt[16 * st + 8 * g + j][wave * 32 + lr];
+                return split3(x, 0);
+            }, wave, lane);
 #pragma unroll
         for (int t4 = 0; t4 < DH; t4 += 4) {
             const f32x4 qq = *reinterpret_cast<const f32x4 *>(&sm.q[lr][g * DH + t4]);
@@ -539,8 +555,7 @@ DEVI void key_tile(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int kt, i
 
 // The steps [i0, i1) of a key tile in plain float32 arithmetic, for key_tile_x3's tiles whose sums
 // were not finite: the wave's accumulator (dV of its keys for the first four waves, dK for the
-// others, in MFMA layout) and the tile's dQ slot rows (with float atomics the shares are in dq
-// already and stay).  Slow and rare.
+// others, in MFMA layout) and the tile's dQ slot rows.  Slow and rare.
 template <int D, bool CAUSAL, int MASK>
 DEVI void redo_key_tile(const BwdArgs &a, int tid, int bhk, int kt, int i0, int i1, f32x16 (&acc)[D / 32]) {
     const AttnShape &s = a.s;
@@ -577,7 +592,7 @@ DEVI void redo_key_tile(const BwdArgs &a, int tid, int bhk, int kt, int i0, int 
         for (int qq = m0; qq < min(m0 + kBM, s.L); ++qq) {
             const int64_t row = (int64_t)bh * s.L + qq;
             // dQ: the waves take the rows in turn, lanes the tile's keys, then lanes the dims.
-            if (a.dq_part && (qq & 7) == wave) {
+            if ((qq & 7) == wave) {
                 float p, d0, d1, t = 0.f;
                 pair(bh, qq, n0 + lane, p, d0);
                 pair(bh, qq, n0 + 64 + lane, p, d1);
@@ -642,7 +657,7 @@ struct alignas(16) BwdSmemX3 {
 // MASK: 0 none, 1 a value per (query, key), 2 the same for every query (key padding).
 template <int D, bool CAUSAL, int MASK, bool VEC>
 DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int kt, int i0, int i1, float *kdst,
-                      float *vdst, bool kv_atomic) {
+                      float *vdst) {
     constexpr int KSTEP = D / 16, NDT = D / 32;
     const AttnShape &s = a.s;
     const int wave8 = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave8 & 3;
@@ -665,11 +680,9 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         if (p.m0 >= s.L) p.m0 = m_begin, ++p.bh;
         return p;
     };
-    const bool dq_atomic = a.dq_part == nullptr;
     const int rf = slot_from(s, kt);
     const int64_t slot0 = slot_before(s, kt) * ((int64_t)s.B * s.H);
     auto dq_dst = [&](Pos p) -> float * {
-        if (dq_atomic) return a.dq_acc + ((int64_t)p.bh * s.L + p.m0) * s.E;
         return a.dq_part + (slot0 + (int64_t)p.bh * (s.L - rf) + (p.m0 - rf)) * s.E;
     };
     // Padding: a wave none of whose keys is visible to any query does no work where that is exact
@@ -714,7 +727,7 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
     const Pos first{b * s.H + hk * s.repeat + (i0 < i1 ? i0 / per_head : 0), m_begin + (i0 < i1 ? i0 % per_head : 0) * kBM};
 
-    // The waves' shares of the dQ of the step at p, added and stored (or added into dq).
+    // The waves' shares of the dQ of the step at p, added and stored.
     auto reduce_dq = [&](Pos p) {
         float *dst = dq_dst(p);
         const int rows = min(kBM, s.L - p.m0);
@@ -725,16 +738,13 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         for (int w = 0; w < kWaves; ++w)
             if (live_at(w, p.m0)) t += *reinterpret_cast<const f32x4 *>(&sm.part[w][r][d]);
         if (r >= rows) return;
-        if (!dq_atomic && (s.E & 3) == 0) {  // slots start 16-byte aligned and rows are whole parts
+        if ((s.E & 3) == 0) {  // slots start 16-byte aligned and rows are whole parts
             if (d < s.E) *reinterpret_cast<f32x4 *>(dst + (int64_t)r * s.E + d) = t;
             return;
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (d + e < s.E) {
-                if (dq_atomic) unsafeAtomicAdd(dst + (int64_t)r * s.E + d + e, t[e] * s.scale);
-                else dst[(int64_t)r * s.E + d + e] = t[e];
-            }
+            if (d + e < s.E) dst[(int64_t)r * s.E + d + e] = t[e];
     };
 
     if (i0 < i1) {
@@ -789,13 +799,11 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             open = __builtin_amdgcn_readfirstlane(all ? seen : 15);
         }
         if (open == 0) {  // nothing visible: the tile's dQ shares are zero
-            if (!dq_atomic) {
-                Pos p = first;
-                for (int i = i0; i < i1; ++i, p = next_pos(p)) {
-                    float *dst = dq_dst(p);
-                    const int count = min(kBM, s.L - p.m0) * s.E;
-                    for (int j = tid; j < count; j += kX3Threads) dst[j] = 0.f;
-                }
+            Pos p = first;
+            for (int i = i0; i < i1; ++i, p = next_pos(p)) {
+                float *dst = dq_dst(p);
+                const int count = min(kBM, s.L - p.m0) * s.E;
+                for (int j = tid; j < count; j += kX3Threads) dst[j] = 0.f;
             }
         } else {
             if (group_a) {
@@ -1015,35 +1023,16 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             float bad = 0.f;
 #pragma unroll
             for (int dt = 0; dt < NDT; ++dt) bad += not_finite(acc[dt]);
-            if (__syncthreads_or(bad != 0.f)) redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+            if (__syncthreads_or(bad != 0.f)) {
+                __syncthreads();  // the dQ slots' first stores are ordered before the second
+                redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+            }
         }
     }
 
     // dV, or dK times scale, of this lane's key.
     const float mul = group_a ? 1.f : s.scale;
     float *tile_dst = group_a ? vdst : kdst;
-    if (kv_atomic) {
-        // A share of the tile's steps, added atomically through LDS: one atomic instruction then
-        // covers consecutive dims of one key (see key_tile).
-        constexpr int RS = D + 4;
-        static_assert(2 * kWaves * 32 * RS * sizeof(float) <= sizeof(BwdSmemX3<D>), "per-wave blocks fit");
-        float *blk = reinterpret_cast<float *>(&sm) + wave8 * 32 * RS;
-        const int rows = min(32, s.S - kw0);
-        __syncthreads();  // the previous readers of the area are done
-#pragma unroll
-        for (int dt = 0; dt < NDT; ++dt)
-#pragma unroll
-            for (int r = 0; r < 16; r += 4)
-                *reinterpret_cast<f32x4 *>(blk + lr * RS + dt * 32 + acc_row(r, g)) =
-                    f32x4{acc[dt][r] * mul, acc[dt][r + 1] * mul, acc[dt][r + 2] * mul, acc[dt][r + 3] * mul};
-        __syncthreads();
-        float *dst = tile_dst + (int64_t)(kw0 - n0) * s.E;
-        for (int i = lane; i < rows * D; i += 64) {
-            const int rr = i / D, d = i % D;
-            if (d < s.E) unsafeAtomicAdd(dst + (int64_t)rr * s.E + d, blk[rr * RS + d]);
-        }
-        return;
-    }
     if (key < s.S) {
         float *dst = tile_dst + (int64_t)(key - n0) * s.E;
 #pragma unroll
@@ -1336,7 +1325,7 @@ DEVI void key_tile_any(const BwdArgs &a, BwdSmem<D> &sm, int tid, int bhk, int k
 }
 
 template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16>
-__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(K16), bwd_waves_per_eu(K16)))) void bwd_f32_kernel(BwdArgs a) {
+__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(D, MASK, K16), bwd_waves_per_eu(D, MASK, K16)))) void bwd_f32_kernel(BwdArgs a) {
     __shared__ BwdSmem<D> sm;
     const int BHk = a.s.B * a.s.Hkv;
     const int kt = blockIdx.x / BHk;  // tile 0 has the most causal work, so it goes first
@@ -1354,7 +1343,7 @@ __global__ __launch_bounds__(kX3Threads) __attribute__((amdgpu_waves_per_eu(2, 2
     const int bhk = blockIdx.x % BHk;
     const int64_t row0 = ((int64_t)bhk * a.s.S + (int64_t)kt * kBN) * a.s.E;
     key_tile_x3<D, CAUSAL, MASK, VEC>(a, sm, threadIdx.x, bhk, kt, 0, tile_steps(a.s, kt),
-                                      static_cast<float *>(a.dk) + row0, static_cast<float *>(a.dv) + row0, false);
+                                      static_cast<float *>(a.dk) + row0, static_cast<float *>(a.dv) + row0);
 }
 
 // Where a stream-K range's share of a key tile it cuts goes: slot 0 of the range for the tile it
@@ -1406,7 +1395,7 @@ DEVI void streamk_range(const BwdArgs &a, const StreamK &sk, F tile) {
 }
 
 template <int D, bool CAUSAL, bool MASK, bool VEC, bool K16>
-__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(K16), bwd_waves_per_eu(K16)))) void bwd_f32_streamk_kernel(BwdArgs a, StreamK sk) {
+__global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_per_eu(bwd_waves_per_eu(D, MASK, K16), bwd_waves_per_eu(D, MASK, K16)))) void bwd_f32_streamk_kernel(BwdArgs a, StreamK sk) {
     __shared__ BwdSmem<D> sm;
     streamk_range(a, sk, [&](int bhk, int kt, int i0, int i1, float *kd, float *vd, bool atomic) {
         key_tile_any<D, CAUSAL, MASK, VEC, K16>(a, sm, threadIdx.x, bhk, kt, i0, i1, kd, vd, atomic);
@@ -1416,8 +1405,8 @@ __global__ __launch_bounds__(layout_threads(K16)) __attribute__((amdgpu_waves_pe
 template <int D, bool CAUSAL, int MASK, bool VEC>
 __global__ __launch_bounds__(kX3Threads) __attribute__((amdgpu_waves_per_eu(2, 2))) void bwd_x3_streamk_kernel(BwdArgs a, StreamK sk) {
     __shared__ BwdSmemX3<D> sm;
-    streamk_range(a, sk, [&](int bhk, int kt, int i0, int i1, float *kd, float *vd, bool atomic) {
-        key_tile_x3<D, CAUSAL, MASK, VEC>(a, sm, threadIdx.x, bhk, kt, i0, i1, kd, vd, atomic);
+    streamk_range(a, sk, [&](int bhk, int kt, int i0, int i1, float *kd, float *vd, bool) {
+        key_tile_x3<D, CAUSAL, MASK, VEC>(a, sm, threadIdx.x, bhk, kt, i0, i1, kd, vd);
     });
 }
 
@@ -1570,7 +1559,7 @@ int resident_workgroups(int D, bool mask) { return device_cus() * (D <= 64 && !m
 // busy (a CU left with one workgroup runs it nearly twice as fast), and the cut tiles' extra
 // prologues and partial dK / dV cost 2-6%: B8 H12 L1024 376 -> 391 us, B16 H16 L1024 828 ->
 // 879 us.  chunks == 0: whole tiles.
-StreamK plan_streamk(const AttnShape &s, int D, bool mask) {
+StreamK plan_streamk(const AttnShape &s, int D, bool mask, bool x3) {
     StreamK k{0, 0, 0};
     const int nkt = (s.S + kBN - 1) / kBN;
     for (int kt = 0; kt < nkt; ++kt) k.per_kvh += tile_steps(s, kt);
@@ -1581,7 +1570,7 @@ StreamK plan_streamk(const AttnShape &s, int D, bool mask) {
     const int64_t last = tiles % slots;  // workgroups of the last, partial wave
     const bool underfilled = s.causal ? tiles <= slots : tiles < slots;
     const bool ragged = !s.causal && tiles < 4 * (int64_t)slots && last > 0 && 4 * last <= 3 * (int64_t)slots;
-    if (underfilled || ragged) k.chunks = D <= 64 ? std::max(device_cus() & ~7, 8) : slots;
+    if (underfilled || ragged) k.chunks = x3 ? std::max(device_cus() & ~7, 8) : slots;
     return k;
 }
 
@@ -1594,14 +1583,14 @@ size_t dq_part_bytes(const AttnShape &s) {
 size_t kv_part_bytes(const StreamK &sk, int E) { return (size_t)sk.chunks * 4 * kBN * E * sizeof(float); }
 size_t align256(size_t n) { return (n + 255) / 256 * 256; }
 
-// Head dims 65 to 128 (float32 MFMA): whole tiles or stream-K ranges.
-template <bool VEC, bool K16>
-hipError_t launch_128(const BwdArgs &a, const StreamK &sk, dim3 grid, hipStream_t st) {
+// The float32 tiles: whole or stream-K ranges.
+template <int D, bool VEC, bool K16>
+hipError_t launch_f32(const BwdArgs &a, const StreamK &sk, dim3 grid, hipStream_t st) {
     const dim3 block(layout_threads(K16));
     auto go = [&](auto causal, auto mask) {
         constexpr bool C = decltype(causal)::value, M = decltype(mask)::value;
-        if (sk.chunks > 0) return launch(bwd_f32_streamk_kernel<128, C, M, VEC, K16>, grid, block, st, a, sk);
-        return launch(bwd_f32_kernel<128, C, M, VEC, K16>, grid, block, st, a);
+        if (sk.chunks > 0) return launch(bwd_f32_streamk_kernel<D, C, M, VEC, K16>, grid, block, st, a, sk);
+        return launch(bwd_f32_kernel<D, C, M, VEC, K16>, grid, block, st, a);
     };
     const std::true_type yes;
     const std::false_type no;
@@ -1626,8 +1615,9 @@ hipError_t launch_tiles(const BwdArgs &a, const StreamK &sk, hipStream_t st) {
     const int nkt = (a.s.S + kBN - 1) / kBN;
     const dim3 grid(sk.chunks > 0 ? sk.chunks : nkt * a.s.B * a.s.Hkv);
     if constexpr (D == 128) {  // the 8-wave tile of 16 keys, or on request the forward-consistent 4-wave tile
-        return a.s.consistent ? launch_128<VEC, false>(a, sk, grid, st) : launch_128<VEC, true>(a, sk, grid, st);
+        return a.s.consistent ? launch_f32<D, VEC, false>(a, sk, grid, st) : launch_f32<D, VEC, true>(a, sk, grid, st);
     } else {
+        if (!a.dq_part) return launch_f32<D, VEC, false>(a, sk, grid, st);
         if (!a.s.mask) return launch_x3<D, 0, VEC>(a, sk, grid, st);
         return a.s.msl == 0 ? launch_x3<D, 2, VEC>(a, sk, grid, st) : launch_x3<D, 1, VEC>(a, sk, grid, st);
     }
@@ -1636,18 +1626,19 @@ hipError_t launch_tiles(const BwdArgs &a, const StreamK &sk, hipStream_t st) {
 template <int D>
 hipError_t launch_d(const BwdArgs &args, size_t part_bytes, hipStream_t st) {
     BwdArgs a = args;
-    // The ABI checked 16-byte alignment; the float32 tiles want E to fill D, the others whole
-    // 16-byte parts of rows.
-    a.s.vec = args.s.vec && (D == 128 ? args.s.E == D : args.s.E % 4 == 0);
-    const StreamK sk = plan_streamk(a.s, D, a.s.mask != nullptr);
-    record_schedule(streamk_ranges, sk.chunks);
+    StreamK sk = plan_streamk(a.s, D, a.s.mask != nullptr, D <= 64);
     // Deterministic when the workspace holds the slots; otherwise float atomics.
     const size_t dq_bytes = align256(dq_part_bytes(a.s));
     if (a.dq_part && dq_bytes + kv_part_bytes(sk, a.s.E) <= part_bytes) {
         a.kv_part = sk.chunks > 0 ? a.dq_part + dq_bytes / sizeof(float) : nullptr;
     } else {
         a.dq_part = a.kv_part = nullptr, a.tame = nullptr;
+        sk = plan_streamk(a.s, D, a.s.mask != nullptr, false);
     }
+    record_schedule(streamk_ranges, sk.chunks);
+    // The ABI checked 16-byte alignment; the float32 tiles want E to fill D, the others whole
+    // 16-byte parts of rows.
+    a.s.vec = args.s.vec && (D == 128 || !a.dq_part ? args.s.E == D : args.s.E % 4 == 0);
     record_schedule(deterministic, a.dq_part ? 1 : 0);
     const int64_t rows = (int64_t)a.s.B * a.s.H * a.s.L;
     const int rows_blocks = (int)((rows + 15) / 16);
@@ -1669,7 +1660,8 @@ hipError_t launch_d(const BwdArgs &args, size_t part_bytes, hipStream_t st) {
 
 template <int D>
 size_t part_bytes_d(const AttnShape &s) {
-    const size_t kv = std::max(kv_part_bytes(plan_streamk(s, D, false), s.E), kv_part_bytes(plan_streamk(s, D, true), s.E));
+    const size_t kv = std::max(kv_part_bytes(plan_streamk(s, D, false, D <= 64), s.E),
+                               kv_part_bytes(plan_streamk(s, D, true, D <= 64), s.E));
     return align256(dq_part_bytes(s)) + align256(kv);
 }
 
