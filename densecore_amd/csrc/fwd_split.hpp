@@ -99,7 +99,8 @@ DEVI void store_out(__bf16 *p, float x) { *p = static_cast<__bf16>(x); }
 
 // Combines the pieces of split query tiles, 16 lanes per query row: with the pieces' lse values
 // l_p and normalized outputs o_p, lse = log sum exp(l_p) and out = sum exp(l_p - lse) o_p.  A row
-// no piece sees any key of keeps the reference's out = 0, lse = 0.  Rows of query tiles that ran
+// no piece sees any key of keeps the reference's out = 0, lse = 0; one whose pieces are NaN (a NaN
+// query) is NaN.  Rows of query tiles that ran
 // whole were written by the forward and are skipped.  Each lane carries 4 consecutive dims of
 // each 64 (16-byte loads when the partial rows' width is a multiple of 4), so a wave merges 4
 // rows with independent loads.
@@ -115,8 +116,9 @@ __global__ __launch_bounds__(256) void fwd_split_merge_kernel(FwdArgs a, int kBM
     const float *po = a.split_o + row * a.split_max * s.E;
     OutT *orow = static_cast<OutT *>(a.out) + row * s.E;
     float mx = -INFINITY;
-    for (int p = 0; p < np; ++p) mx = fmaxf(mx, pl[p]);
-    if (mx == -INFINITY) {
+    bool nan = false;
+    for (int p = 0; p < np; ++p) mx = fmaxf(mx, pl[p]), nan |= pl[p] != pl[p];
+    if (mx == -INFINITY && !nan) {
         for (int d = sub; d < s.E; d += 16) store_out(orow + d, 0.f);
         if (sub == 0) a.lse[row] = 0.f;
         return;

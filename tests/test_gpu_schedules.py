@@ -25,7 +25,7 @@ others stream-K.  Tolerance, as for every float32 output: |gpu - ref| <= 2e-5 + 
 import numpy as np
 import pytest
 
-from tests._data import assert_bf16, assert_f32, bf16_round
+from tests._data import assert_bf16, assert_bf16_nan, assert_f32, assert_f32_nan, bf16_round
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -272,3 +272,21 @@ def test_split_shapes_without_split_workspace(oracle_lib, dtype):
         ref = oracle_lib.backward(g, q, k, v, ref_o, ref_l, causal)
     for name, a, b in zip(("dq", "dk", "dv"), (dq, dk, dv), ref):
         check(a.float().cpu().numpy(), b, f"{dtype} {name}, reduced workspace")
+
+
+@pytest.mark.parametrize("bf16,E", [(False, 64), (False, 128), (True, 128)])
+def test_split_forward_of_a_nan_query(oracle_lib, bf16, E):
+    """A query that is NaN in every piece of a split key range is NaN, as in a whole one."""
+    from densecore_amd import _native
+    print(f"[case] split forward of a NaN query bf16={bf16} E{E}", flush=True)
+    rng = np.random.default_rng(E)
+    q, k, v = (bf16_round(rng.standard_normal((1, 2, 2048, E), dtype=np.float32)) for _ in range(3))
+    q[0, 1, 70, 3] = np.nan
+    ref_o, ref_l = oracle_lib.forward(q, k, v, False)
+    t = [_t(x).to(torch.bfloat16) if bf16 else _t(x) for x in (q, k, v)]
+    assert _native._schedule(False, *t, False)["split_pieces"] > 1
+    out, lse = _native._flash_attention(*t, False)
+    out, lse = out.float().cpu().numpy(), lse.cpu().numpy()
+    assert np.isnan(ref_o[0, 1, 70]).all() and np.isnan(ref_l[0, 1, 70])
+    (assert_bf16_nan if bf16 else assert_f32_nan)(out, ref_o, "out")
+    (assert_bf16_nan if bf16 else assert_f32_nan)(lse, ref_l, "lse")
