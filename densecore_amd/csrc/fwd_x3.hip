@@ -99,20 +99,21 @@ __attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd(D), fwd_waves_per_simd(D))
     const int t_end = SPLIT ? (piece + 1) * ntiles / npieces : ntiles;
 
     // Row masks: the tiles with any visible key, listed, so that the others (padding) are neither
-    // staged nor computed.  (Rows of more tiles than the list holds go through all of them.)
-    const bool listed = LIST && ntiles <= kOrderMaxTiles;
+    // staged nor computed; kOrderMaxTiles tiles from w0 on at a time.
+    int w0 = 0;
     int n = t_end - t_begin;
-    if (listed) {
-        for (int seg = wave; seg * 64 < s.S; seg += kX3Waves) {
+    auto list_tiles = [&]() {
+        const int w1 = min(ntiles, w0 + kOrderMaxTiles);
+        for (int seg = w0 / 2 + wave; 2 * seg < w1; seg += kX3Waves) {
             const int key = seg * 64 + lane;
             const uint64_t open = __ballot(key < s.S && mrow[key] != -INFINITY);
-            if (lane < 2 && 2 * seg + lane < ntiles) open_tile[2 * seg + lane] = ((open >> (32 * lane)) & 0xffffffffull) != 0;
+            if (lane < 2 && 2 * seg + lane < w1) open_tile[2 * seg + lane - w0] = ((open >> (32 * lane)) & 0xffffffffull) != 0;
         }
         __syncthreads();
         if (wave == 0) {
             int count = 0;
-            for (int t0 = 0; t0 < ntiles; t0 += 64) {
-                const bool open = t0 + lane < ntiles && open_tile[t0 + lane] != 0;
+            for (int t0 = 0; t0 < w1 - w0; t0 += 64) {
+                const bool open = t0 + lane < w1 - w0 && open_tile[t0 + lane] != 0;
                 const uint64_t set = __ballot(open);
                 if (open) list[count + __popcll(set & ((1ull << lane) - 1))] = (uint16_t)(t0 + lane);
                 count += __popcll(set);
@@ -121,18 +122,20 @@ __attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd(D), fwd_waves_per_simd(D))
         }
         __syncthreads();
         n = list_len;
-    }
+    };
+    if constexpr (LIST) list_tiles();
     n = __builtin_amdgcn_readfirstlane(n);
-    auto key0 = [&](int i) { return (listed ? __builtin_amdgcn_readfirstlane((int)list[i]) : t_begin + i) * BN; };
+    auto key0 = [&](int i) { return (LIST ? w0 + __builtin_amdgcn_readfirstlane((int)list[i]) : t_begin + i) * BN; };
 
     // The first tiles' loads go out before the queries are split.
     X3Stage<BN, D, kX3Threads, VEC> kst, vst;
     X3Stage<BN, D, kX3Threads, VEC> k1;
-    if (n > 0) {
+    auto load_first = [&]() {
         kst.load(kb, key0(0), s.S - 1, s.E, tid);
         vst.load(vb, key0(0), s.S - 1, s.E, tid);
         k1.load(kb, key0(min(1, n - 1)), s.S - 1, s.E, tid);
-    }
+    };
+    if (n > 0) load_first();
     // Without a mask the scale is applied after the tile max and inside each exponent's FMA: for a
     // positive scale the max of the rounded products equals the rounded product of the max, and the
     // exponent is rounded once instead of twice.  A negative scale enters as its magnitude with the
@@ -332,22 +335,35 @@ __attribute__((amdgpu_waves_per_eu(fwd_waves_per_simd(D), fwd_waves_per_simd(D))
                 settle(i + 1, sacc, mcur);
             }
         };
-        if (n > 0) {
-            kst.store(sk[0], tid);
-            vst.store(sv[0], tid);
-            k1.store(sk[1], tid);
-            if (n > 2) kst.load(kb, key0(2), s.S - 1, s.E, tid);
-            if (n > 1) vst.load(vb, key0(1), s.S - 1, s.E, tid);
-            if constexpr (MASK == kRowMask) mcur = row_mask(0), mnext = row_mask(min(1, n - 1));
-            __syncthreads();
-            if (wlast >= 0) {
-                scores(0, sacc);
-                settle(0, sacc, mcur);
+        for (;;) {
+            if (n > 0) {
+                kst.store(sk[0], tid);
+                vst.store(sv[0], tid);
+                k1.store(sk[1], tid);
+                if (n > 2) kst.load(kb, key0(2), s.S - 1, s.E, tid);
+                if (n > 1) vst.load(vb, key0(1), s.S - 1, s.E, tid);
+                if constexpr (MASK == kRowMask) mcur = row_mask(0), mnext = row_mask(min(1, n - 1));
+                __syncthreads();
+                if (wlast >= 0) {
+                    scores(0, sacc);
+                    settle(0, sacc, mcur);
+                }
+                const int steady = min(wlast, n - 2);
+                int i = 0;
+                for (; i < steady; ++i) step(i, std::true_type{});
+                for (; i < n; ++i) step(i, std::false_type{});
             }
-            const int steady = min(wlast, n - 2);
-            int i = 0;
-            for (; i < steady; ++i) step(i, std::true_type{});
-            for (; i < n; ++i) step(i, std::false_type{});
+            if constexpr (LIST) {
+                w0 += kOrderMaxTiles;
+                if (w0 >= ntiles) break;
+                __syncthreads();  // everyone is done with the list and the last tiles
+                list_tiles();
+                n = __builtin_amdgcn_readfirstlane(n);
+                wlast = n - 1;
+                if (n > 0) load_first();
+            } else {
+                break;
+            }
         }
     } else {
         // A mask value per (query, key): tiles one after the other, a tile whose mask is -inf for
