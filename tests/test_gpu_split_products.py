@@ -9,7 +9,7 @@ plain float32 arithmetic.
 import numpy as np
 import pytest
 
-from tests._data import assert_f32
+from tests._data import assert_f32, assert_f32_nan
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
@@ -122,3 +122,58 @@ def test_infinite_output_gradient():
     assert np.isposinf(dv[0, 1, :, 9]).all()
     assert_f32(np.delete(dv[0, 1], 9, -1), np.delete(dv0[0, 1], 9, -1), "other dims")
     assert_f32(dv[0, 0], dv0[0, 0], "other head")
+
+
+@pytest.mark.parametrize("E,causal,mask", [(64, True, None), (40, False, "pad"), (33, False, None), (80, True, "full")])
+def test_nan_is_final(oracle_lib, E, causal, mask):
+    """NaN in one key, one value and one query: NaN where the oracle has it, the bar elsewhere, in a
+    multiple of the time (121 times when the rows a NaN reaches were computed again in float32, now 1.3);
+    with an element beyond the split beside them too."""
+    from densecore_amd import _native
+    print(f"[case] NaN operands E{E} causal={causal} mask={mask}", flush=True)
+    rng = np.random.default_rng(E)
+    B, H, L = 2, 3, 300
+    q, k, v = (rng.standard_normal((B, H, L, E), dtype=np.float32) for _ in range(3))
+    m = _mask(mask, rng, B, H, L, L)
+    if mask == "pad":
+        m[:] = 0
+        m[1, ..., 200:] = -np.inf
+    full = None if m is None else np.ascontiguousarray(np.broadcast_to(m, (B, H, L, L)))
+    tm = None if m is None else _t(m).expand(B, H, L, L)
+    q[0, 1, 7, 3] = k[0, 2, 150, 1] = v[1, 0, 20, 2] = np.nan
+    for beyond in (False, True):
+        if beyond:
+            v[0, 1, 9, 5] = 3e38
+        with np.errstate(all="ignore"):
+            ref_o, ref_l = oracle_lib.forward(q, k, v, causal, None, full)
+        out, lse = _native._flash_attention(_t(q), _t(k), _t(v), causal, None, tm)
+        out, lse = out.cpu().numpy(), lse.cpu().numpy()
+        if beyond:  # relative to the element's size
+            assert np.allclose(out[0, 1, :, 5] / 3e38, ref_o[0, 1, :, 5] / 3e38, rtol=1e-4, atol=2e-5, equal_nan=True)
+            out, ref_o = np.delete(out, 5, -1), np.delete(ref_o, 5, -1)
+        assert_f32_nan(out, ref_o, "out")
+        assert_f32_nan(lse, ref_l, "lse")
+
+
+def test_nan_takes_no_longer():
+    from densecore_amd import _native
+    gen = torch.Generator(device=DEV).manual_seed(2)
+    q, k, v = (torch.randn(8, 12, 1024, 64, generator=gen, device=DEV) for _ in range(3))
+
+    def us():
+        _native._flash_attention(q, k, v, True)
+        times = []
+        for _ in range(4):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            start.record()
+            _native._flash_attention(q, k, v, True)
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end) * 1e3)
+        return min(times)
+
+    plain = us()
+    k[:, :, 5] = float("nan")
+    after = us()
+    print(f"  {plain:.0f} us, with NaN {after:.0f} us", flush=True)
+    assert after < 10 * plain
