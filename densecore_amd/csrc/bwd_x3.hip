@@ -150,7 +150,8 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
     auto look = [&](bool &any, bool &tame) {  // this wave's part
         any = __any(key < s.S && mbase[min(key, s.S - 1)] != -INFINITY);
         tame = true;
-        for (int j = tid; j < (i1 - i0) * kBM; j += kX3Threads) {
+        const int ltid = opaque_index(tid), llane = ltid & 63;
+        for (int j = ltid; j < (i1 - i0) * kBM; j += kX3Threads) {
             const int i = i0 + j / kBM, qq = m_begin + (i % per_head) * kBM + j % kBM;
             if (qq < s.L) tame &= a.tame[(int64_t)(b * s.H + hk * s.repeat + i / per_head) * s.L + qq] != 0;
         }
@@ -159,14 +160,14 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             const int count = min(32, s.S - kw0) * s.E;
             if constexpr (VEC) {
 #pragma unroll 8
-                for (int j = 4 * lane; j < count; j += 256) {
+                for (int j = 4 * llane; j < count; j += 256) {
                     const f32x4 x = *reinterpret_cast<const f32x4 *>(rows + j);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) tame &= fabsf(x[e]) <= kTame;
                 }
             } else {
 #pragma unroll 8
-                for (int j = lane; j < count; j += 64) tame &= fabsf(rows[j]) <= kTame;
+                for (int j = llane; j < count; j += 64) tame &= fabsf(rows[j]) <= kTame;
             }
         }
         tame = __all(tame);
@@ -187,7 +188,8 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
     auto reduce_dq = [&](Pos p) {
         float *dst = dq_dst(p);
         const int rows = min(kBM, s.L - p.m0);
-        const int r = tid / (D / 4), d = tid % (D / 4) * 4;
+        const int otid = opaque_index(tid);
+        const int r = otid / (D / 4), d = otid % (D / 4) * 4;
         if (kBM * D / 4 < kX3Threads && tid >= kBM * D / 4) return;
         f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -231,14 +233,14 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
         static_assert(kWaves * sizeof(X3Tile<kBM, D>) <= sizeof(sm.ds) + sizeof(sm.part), "the rows fit");
         X3Tile<kBM, D> &wt = reinterpret_cast<X3Tile<kBM, D> *>(&sm.ds[0])[wave];
         X3Stage<kBM, D, 64, VEC> rows;
-        rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, lane);
+        rows.load((static_cast<const float *>(group_a ? a.k : a.v)) + (int64_t)bhk * s.S * s.E, kw0, s.S - 1, s.E, opaque_index(lane));
         load_step();
         bool any = true, tame = true;
         if (MASK == 2 && a.tame) look(any, tame);
         __syncthreads();  // a previous tile's last readers of these areas are done
         if (MASK == 2 && lane == 0) sm.seen[wave8] = (any ? 1 : 0) | (tame ? 2 : 0);
         if (group_a) {
-            rows.store(wt, lane);
+            rows.store(wt, opaque_index(lane));
             store_do(0);
         } else {
             stage.store(sm.q[0], gtid);
@@ -273,7 +275,7 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             }
             __syncthreads();
             if (!group_a) {
-                rows.store(wt, lane);
+                rows.store(wt, opaque_index(lane));
                 __builtin_amdgcn_wave_barrier();
 #pragma unroll
                 for (int st = 0; st < KSTEP; ++st) kv[st] = row_frag_x3(wt, rowb, 0, st);
@@ -481,7 +483,7 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
             for (int dt = 0; dt < NDT; ++dt) bad += not_finite(acc[dt]);
             if (__syncthreads_or(bad != 0.f)) {
                 __syncthreads();  // the dQ slots' first stores are ordered before the second
-                redo_key_tile<D, CAUSAL, MASK>(a, tid, bhk, kt, i0, i1, acc);
+                redo_key_tile<D, CAUSAL, MASK>(a, opaque_index(tid), bhk, kt, i0, i1, acc);
             }
         }
     }
@@ -489,13 +491,14 @@ DEVI void key_tile_x3(const BwdArgs &a, BwdSmemX3<D> &sm, int tid, int bhk, int 
     // dV, or dK times scale, of this lane's key.
     const float mul = group_a ? 1.f : s.scale;
     float *tile_dst = group_a ? vdst : kdst;
-    if (key < s.S) {
-        float *dst = tile_dst + (int64_t)(key - n0) * s.E;
+    const int etid = opaque_index(tid), ekey = kw0 + (etid & 31), eg = (etid & 63) >> 5;
+    if (ekey < s.S) {
+        float *dst = tile_dst + (int64_t)(ekey - n0) * s.E;
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
             for (int r = 0; r < 16; r += 4) {
-                const int d = dt * 32 + acc_row(r, g);
+                const int d = dt * 32 + acc_row(r, eg);
                 if (VEC) {
                     if (d < s.E)
                         *reinterpret_cast<f32x4 *>(dst + d) =
