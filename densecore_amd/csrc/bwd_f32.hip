@@ -923,14 +923,12 @@ __global__ __launch_bounds__(256) void bwd_reduce_f32_kernel(BwdArgs a, StreamK 
     }
 }
 
-// The slots the schedules below were measured on: two workgroups per CU at D <= 64 without a mask,
-// one otherwise; 0 if unknown.  (key_tile_x3 runs one per CU at every D <= 64; the lines between the
-// schedules hold for it too, but it is given one range per CU: two cost a second prologue each,
-// causal B5 H16 L241 D64 61.8 against 51.5 us, B1 H12 L521 62.0 against 43.7.)
+// Workgroups of the float32 tiles that fit on the device at once: two per CU at D <= 64 without a
+// mask, one otherwise; 0 if unknown.
 int resident_workgroups(int D, bool mask) { return device_cus() * (D <= 64 && !mask ? 2 : 1); }
 
-// The stream-K schedule where whole tiles leave part of the device idle (measured on one MI355X,
-// dc_sdpa_bwd per call, whole tiles -> stream-K):
+// The stream-K schedule where whole tiles leave part of the device idle; chunks == 0: whole tiles.
+// The float32 tiles (measured on one MI355X, dc_sdpa_bwd per call, whole tiles -> stream-K):
 //   * fewer key tiles than resident workgroups, or (causal, tiles of unequal work) as many:
 //     causal B1 H8 L2048 D64 405 -> 137 us, B1 H4 L8192 1592 -> 742 us, B8 H12 L512 149 -> 128
 //     us, B2 H16 L1024 D128 (256 tiles, 256 slots) 454 -> 315 us;
@@ -939,19 +937,40 @@ int resident_workgroups(int D, bool mask) { return device_cus() * (D <= 64 && !m
 // With at least as many causal tiles as slots, whole tiles dealt longest first keep the device
 // busy (a CU left with one workgroup runs it nearly twice as fast), and the cut tiles' extra
 // prologues and partial dK / dV cost 2-6%: B8 H12 L1024 376 -> 391 us, B16 H16 L1024 828 ->
-// 879 us.  chunks == 0: whole tiles.
+// 879 us.
+//
+// key_tile_x3 (x3) runs one workgroup per CU and is given one range per CU (two cost a second prologue
+// each, causal B5 H16 L241 D64 61.8 against 51.5 us).  Up to two workgroups' worth of tiles per CU the
+// lines are its own (D64, 256 CUs; whole tiles / stream-K, us):
+//   * causal tiles, as many as CUs at most: L1024, 160 tiles 116 / 73, 256 121 / 100, 320 124 / 125, 384
+//     128 / 141, 512 155 / 175; L4096, 256 427 / 291, 384 456 / 424, 512 525 / 560; L512, 160 80 / 69,
+//     256 83 / 87, 320 86 / 111; L256 (8 steps at most) 41 / 43 at 160;
+//   * equal tiles, up to 5/8 of the CUs or a last wave half full at most: L500, 120 tiles 64 / 56, 200 68 /
+//     77, 240 72 / 86, 264 126 / 94, 384 130 / 121, 416 132 / 135, 480 138 / 152; L2048, 160 216 / 176, 256
+//     250 / 259; a mask per (query, key), 320 156 / 131, 384 157 / 150;
+//   * under key padding tiles are of unequal work, closed ones nearly free, and fill the second wave by
+//     themselves: 160 tiles 70 / 69, 320 96 / 108, 384 133 / 123.
+// Beyond, the float32 tiles' lines are kept; there the two differ by less: 560 tiles 195 / 178, 640 198 /
+// 194, 700 204 / 216, 768 216 / 228, 820 264 / 255, 900 270 / 276, 1400 415 / 427.
 StreamK plan_streamk(const AttnShape &s, int D, bool mask, bool x3) {
     StreamK k{0, 0, 0};
     const int nkt = (s.S + kBN - 1) / kBN;
     for (int kt = 0; kt < nkt; ++kt) k.per_kvh += tile_steps(s, kt);
     k.total = k.per_kvh * s.B * s.Hkv;
-    const int slots = resident_workgroups(D, mask) & ~7;
+    const int slots = resident_workgroups(D, mask) & ~7, cus = device_cus() & ~7;
     if (slots < 8 || k.total == 0) return k;
     const int64_t tiles = (int64_t)nkt * s.B * s.Hkv;
+    if (x3 && tiles <= 2 * (int64_t)cus) {
+        const bool padding = mask && s.msl == 0 && s.msh == 0;
+        const bool few = s.causal ? tiles <= cus : 8 * tiles <= 5 * (int64_t)cus;
+        const bool second = !s.causal && !padding && tiles > cus && 2 * tiles <= 3 * (int64_t)cus;
+        if (few || second) k.chunks = cus;
+        return k;
+    }
     const int64_t last = tiles % slots;  // workgroups of the last, partial wave
     const bool underfilled = s.causal ? tiles <= slots : tiles < slots;
     const bool ragged = !s.causal && tiles < 4 * (int64_t)slots && last > 0 && 4 * last <= 3 * (int64_t)slots;
-    if (underfilled || ragged) k.chunks = x3 ? std::max(device_cus() & ~7, 8) : slots;
+    if (underfilled || ragged) k.chunks = x3 ? cus : slots;
     return k;
 }
 
