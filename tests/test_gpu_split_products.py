@@ -177,3 +177,39 @@ def test_nan_takes_no_longer():
     after = us()
     print(f"  {plain:.0f} us, with NaN {after:.0f} us", flush=True)
     assert after < 10 * plain
+
+
+@pytest.mark.parametrize("exponent", [-60, -100])
+def test_small_magnitudes(exponent):
+    """The parts of a value of 2^-110 and above are bf16 numbers, subnormal ones among them, which the
+    matrix cores do not flush: V, dO and a product's operand scaled down by a power of two give the
+    scaled results, as far from float64 as unscaled ones.  (Below, what a part loses is under 2^-133; dS
+    is smaller than dO by the probabilities, so dQ and dK are held at the larger scale.)"""
+    from densecore_amd import _native
+    rng = np.random.default_rng(7)
+    scale = np.float32(2.0 ** exponent)
+    q, k, v, g = (rng.standard_normal((1, 2, 200, 64), dtype=np.float32) for _ in range(4))
+    x64 = [x.astype(np.float64) for x in (q, k, v, g)]
+    p = np.einsum("bhle,bhse->bhls", x64[0], x64[1]) / 8
+    p = np.exp(p - p.max(-1, keepdims=True))
+    p /= p.sum(-1, keepdims=True)
+    o64 = p @ x64[2]
+    dp = np.einsum("bhle,bhse->bhls", x64[3], x64[2])
+    ds = p * (dp - (x64[3] * o64).sum(-1, keepdims=True)) / 8
+    want = {"out": o64, "dq": ds @ x64[1], "dk": np.einsum("bhls,bhle->bhse", ds, x64[0]),
+            "dv": np.einsum("bhls,bhle->bhse", p, x64[3]), "bmm": np.einsum("bhle,bhse->bhls", x64[2], x64[1])[0]}
+
+    def errors(s):
+        out, lse = _native._flash_attention(_t(q), _t(k), _t(v), False)
+        got = {"out": _native._flash_attention(_t(q), _t(k), _t(v * s), False)[0]}
+        grads = _native._flash_attention_backward(_t(g * s), _t(q), _t(k), _t(v), out, lse, False)
+        got.update(zip(("dq", "dk", "dv"), grads))
+        got["bmm"] = _native._bmm(_t((v * s)[0]), _t(k[0]).transpose(1, 2))
+        return {n: np.linalg.norm(a.cpu().numpy().astype(np.float64) / s - want[n]) / np.linalg.norm(want[n]) for n, a in got.items()}
+
+    plain, small = errors(np.float32(1)), errors(scale)
+    print(f"  {plain}\n  {small}", flush=True)
+    for n in want:
+        if exponent < -90 and n in ("dq", "dk"):
+            continue
+        assert small[n] <= 1.05 * plain[n], n
