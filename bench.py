@@ -31,7 +31,6 @@ import numpy as np
 HERE = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, HERE)
 
-PEAK_FP32_MFMA = 157.3   # TFLOP/s, MI355X dense
 # Float32 products on the bf16 matrix cores: six products per float32 one (2500 / 6).
 PEAK_FP32_SPLIT = 2500.0 / 6
 PEAK_BF16_MFMA = 2500.0  # TFLOP/s, MI355X dense
@@ -338,7 +337,7 @@ def bench_math(torch, steps, warmup, dev):
         res["bmm"][name] = {"dc_bmm_ms": round(ms_dc, 4), "dc_bmm_tflops": round(work / (ms_dc * 1e-3) / 1e12, 2),
                             "hipblaslt_ms": round(ms_bl, 4),
                             "hipblaslt_tflops": round(work / (ms_bl * 1e-3) / 1e12, 2),
-                            "frac_fp32_mfma": round(work / (ms_dc * 1e-3) / 1e12 / PEAK_FP32_MFMA, 4)}
+                            "frac_split_mfma": round(work / (ms_dc * 1e-3) / 1e12 / PEAK_FP32_SPLIT, 4)}
     del qa, ka, wa, va
     q, k, v = (torch.from_numpy(d[c]).to(dev).requires_grad_(True) for c in "qkv")
     am = torch.from_numpy(d["mask_bool"]).to(dev)

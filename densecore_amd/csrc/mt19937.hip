@@ -18,8 +18,9 @@
 //             window follows an update even when the block is a freshly seeded one);
 //   chunks    chunk c covers elements [Eh + c J/2, Eh + (c + 1) J/2), J = 2^17 words; its window
 //             is W(A0 + c J), reached from W(A0) through a radix-64 tree of jumps (c = 64 c1 + c0:
-//             a jump by c1 2^23, then one by c0 2^17; mt_jump_kernel), and one wave generates its
-//             words from that window (mt_chunk_kernel).
+//             a jump by c1 2^23, then one by c0 2^17; mt_jump_kernel), and a workgroup of four
+//             waves takes it from there: two generate its words from that window, two temper and
+//             test them (mt_chunk_kernel).
 // Keep bits: element e is bit e % 32 of word e / 32 (heads and chunks write whole words).  The
 // engine block that holds the last output drawn is written back to the state (by the base
 // workgroup or by the chunk whose range holds the block's first word), and the host moves
