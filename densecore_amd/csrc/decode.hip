@@ -531,7 +531,10 @@ hipError_t launch_dtype(const DecodeArgs &a, hipStream_t st) {
 // workgroup's partials are HG heads wide, so short ranges make the merge the larger part (bf16 B2
 // H32 Hkv4 S16000 D128: 125 splits 55 us, 32 splits 24.5 us; B16 H32 Hkv8 S8192: 2K workgroups 103,
 // 4K 106, 8K 148 us).  The splits are also held to what the scratch of the allocation-free entry
-// point takes, so that it refuses no call for having grouped heads.
+// point takes, so that it refuses no call for having grouped heads; with a workspace too, because both
+// entry points give the same bits.  It binds at batch * heads * head dim in the millions, where workgroups
+// are plenty (B188 H64 Hkv8 S1000 E256 bf16, 1 split or the 2 of a larger scratch: 298.3 us both; B16
+// H128 Hkv8 S2000 E256 float32 189 both).
 int decode_splits(const AttnShape &s, bool bf16, int *split_len) {
     const int64_t BH = (int64_t)s.B * s.H;
     const int64_t max_splits = (s.S + 63) / 64;
