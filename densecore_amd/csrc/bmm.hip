@@ -30,12 +30,16 @@ constexpr int kThreads = 256;
 constexpr int BK = 16;  // one MFMA's depth
 
 // How an operand's tile is loaded: CONTIG_K: 16-byte loads along k; CONTIG_MN: 16-byte loads along
-// m (A) or n (B); SCALAR: one element at a time, any strides.
+// m (A) or n (B); SCALAR: one element at a time, any strides.  RAGGED: the two operands' loads are
+// 4-byte aligned only and the last of a row may be cut short (rows of a length that is not a multiple of
+// 4: loads of one element each took 256 items of 511 x 64 x 511 259 us and, A transposed, 151; now 114
+// and 90).
 enum Layout { CONTIG_K = 0, CONTIG_MN = 1, SCALAR = 2 };
+typedef f32x4 f32x4_ragged __attribute__((aligned(4)));
 
 // One operand's tile: R rows (m or n) by BK, as three chunk-major bf16 planes (x3.hpp), its chunks
 // of 8 along the dimension it is loaded along.
-template <int R, int L>
+template <int R, int L, bool RAGGED>
 struct Operand {
     static constexpr bool ALONG_K = L != CONTIG_MN;
     typedef X3Tile<ALONG_K ? R : BK, ALONG_K ? BK : R> Tile;
@@ -51,6 +55,18 @@ struct Operand {
         r = ((tid >> 1) & 3) + 4 * (grp / (Shape::C / 2));
         return CHUNKS == kThreads || tid < CHUNKS;
     }
+    // Four elements from q on, `left` (at least one) of which exist.
+    DEVI static void part(f32x4 &y, const float *q, int left) {
+        if (!RAGGED) {
+            y = *reinterpret_cast<const f32x4 *>(q);
+        } else if (left >= 4) {
+            y = *reinterpret_cast<const f32x4_ragged *>(q);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (e < left) y[e] = q[e];
+        }
+    }
     // From `p` (the batch item's base) with strides (s_r along the rows, s_k along k); rows past
     // `rows` and k past `kk` read zero.
     DEVI void load(const float *p, int64_t s_r, int64_t s_k, int r0, int rows, int k0, int kk, int tid) {
@@ -61,10 +77,10 @@ struct Operand {
             x[h] = f32x4{0.f, 0.f, 0.f, 0.f};
             if constexpr (L == CONTIG_K) {
                 const int k = k0 + 8 * c + 4 * h;
-                if (r0 + r < rows && k < kk) x[h] = *reinterpret_cast<const f32x4 *>(p + (r0 + r) * s_r + k);
+                if (r0 + r < rows && k < kk) part(x[h], p + (r0 + r) * s_r + k, kk - k);
             } else if constexpr (L == CONTIG_MN) {
                 const int rr = r0 + 8 * c + 4 * h;
-                if (rr < rows && k0 + r < kk) x[h] = *reinterpret_cast<const f32x4 *>(p + (k0 + r) * s_k + rr);
+                if (rr < rows && k0 + r < kk) part(x[h], p + (k0 + r) * s_k + rr, rows - rr);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -106,13 +122,13 @@ struct Operand {
 // Three workgroups per CU, two where the 128 x 128 tile reads an operand transposed (their registers).
 constexpr int waves_per_simd(int BN, int LA, int LB) { return BN == 128 && (LA == CONTIG_MN || LB == CONTIG_MN) ? 2 : 3; }
 
-template <int BM, int BN, int LA, int LB>
+template <int BM, int BN, int LA, int LB, bool RAGGED>
 __global__ __launch_bounds__(kThreads)
 __attribute__((amdgpu_waves_per_eu(waves_per_simd(BN, LA, LB), waves_per_simd(BN, LA, LB)))) void bmm_f32_kernel(BmmArgs g) {
     constexpr int TM = BM / 64, TN = BN / 64;  // 32 x 32 MFMA tiles per wave along m, n
     static_assert(TM >= 1 && TN >= 1, "a wave covers at least 32 x 32");
-    typedef Operand<BM, LA> OpA;
-    typedef Operand<BN, LB> OpB;
+    typedef Operand<BM, LA, RAGGED> OpA;
+    typedef Operand<BN, LB, RAGGED> OpB;
     __shared__ typename OpA::Tile ta[2];
     __shared__ typename OpB::Tile tb[2];
     const int tid = threadIdx.x, lane = tid & 63, lr = lane & 31, gh = lane >> 5;
@@ -262,36 +278,45 @@ __attribute__((amdgpu_waves_per_eu(waves_per_simd(BN, LA, LB), waves_per_simd(BN
 
 bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// The load layout of an operand: contig (the stride that is 1), its extent along that dimension,
-// and the other strides must all keep 16-byte chunks aligned.
-int layout_a(const BmmArgs &g) {
-    if (!aligned16(g.a) || g.sab % 4) return SCALAR;
-    if (g.sak == 1 && g.k % 4 == 0 && g.sam % 4 == 0) return CONTIG_K;
-    if (g.sam == 1 && g.m % 4 == 0 && g.sak % 4 == 0) return CONTIG_MN;
-    return SCALAR;
-}
-int layout_b(const BmmArgs &g) {
-    if (!aligned16(g.b) || g.sbb % 4) return SCALAR;
-    if (g.sbk == 1 && g.k % 4 == 0 && g.sbn % 4 == 0) return CONTIG_K;
-    if (g.sbn == 1 && g.n % 4 == 0 && g.sbk % 4 == 0) return CONTIG_MN;
+// The load layout of an operand: along the dimension whose stride is 1 (`whole`: its extent and the
+// other strides keep 16-byte loads whole and aligned).
+int layout(const float *p, int64_t sb, int64_t s_r, int rows, int64_t s_k, int kk, bool &whole) {
+    const bool along_k = s_k == 1, along_r = s_r == 1;
+    whole = whole && aligned16(p) && sb % 4 == 0;
+    if (along_k && (!along_r || kk > 1)) {
+        whole = whole && kk % 4 == 0 && s_r % 4 == 0;
+        return CONTIG_K;
+    }
+    if (along_r) {
+        whole = whole && rows % 4 == 0 && s_k % 4 == 0;
+        return CONTIG_MN;
+    }
     return SCALAR;
 }
 
+template <int BM, int BN, int LA, int LB>
+hipError_t launch_r(const BmmArgs &g, bool whole, dim3 grid, hipStream_t st) {
+    if constexpr (LA != SCALAR && LB != SCALAR)
+        if (whole) return launch(bmm_f32_kernel<BM, BN, LA, LB, false>, grid, dim3(kThreads), st, g);
+    return launch(bmm_f32_kernel<BM, BN, LA, LB, true>, grid, dim3(kThreads), st, g);
+}
+
 template <int BM, int BN, int LA>
-hipError_t launch_b(const BmmArgs &g, int lb, dim3 grid, hipStream_t st) {
-    if (lb == CONTIG_K) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_K>, grid, dim3(kThreads), st, g);
-    if (lb == CONTIG_MN) return launch(bmm_f32_kernel<BM, BN, LA, CONTIG_MN>, grid, dim3(kThreads), st, g);
-    return launch(bmm_f32_kernel<BM, BN, LA, SCALAR>, grid, dim3(kThreads), st, g);
+hipError_t launch_b(const BmmArgs &g, int lb, bool whole, dim3 grid, hipStream_t st) {
+    if (lb == CONTIG_K) return launch_r<BM, BN, LA, CONTIG_K>(g, whole, grid, st);
+    if (lb == CONTIG_MN) return launch_r<BM, BN, LA, CONTIG_MN>(g, whole, grid, st);
+    return launch_r<BM, BN, LA, SCALAR>(g, whole, grid, st);
 }
 
 template <int BM, int BN>
 hipError_t launch_t(const BmmArgs &g, hipStream_t st) {
     const int64_t tiles = (int64_t)((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN) * g.batch;
     const dim3 grid((unsigned)tiles);
-    const int la = layout_a(g), lb = layout_b(g);
-    if (la == CONTIG_K) return launch_b<BM, BN, CONTIG_K>(g, lb, grid, st);
-    if (la == CONTIG_MN) return launch_b<BM, BN, CONTIG_MN>(g, lb, grid, st);
-    return launch_b<BM, BN, SCALAR>(g, lb, grid, st);
+    bool whole = true;
+    const int la = layout(g.a, g.sab, g.sam, g.m, g.sak, g.k, whole), lb = layout(g.b, g.sbb, g.sbn, g.n, g.sbk, g.k, whole);
+    if (la == CONTIG_K) return launch_b<BM, BN, CONTIG_K>(g, lb, whole, grid, st);
+    if (la == CONTIG_MN) return launch_b<BM, BN, CONTIG_MN>(g, lb, whole, grid, st);
+    return launch_b<BM, BN, SCALAR>(g, lb, whole, grid, st);
 }
 
 // Zeroes C when k == 0 (the reference returns zeros); C is (batch, m, n) through its strides.

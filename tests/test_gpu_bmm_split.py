@@ -87,3 +87,28 @@ def test_nan_rows_are_final():
     a[3, 40, 7] = 3.4e38
     want = (a[3, 40].astype(np.float64) @ b[3].astype(np.float64)).astype(np.float32)
     assert np.allclose(got[40], want, rtol=1e-5) and np.isnan(got[5::128]).all() and np.isfinite(np.delete(got, np.s_[5::128], 0)).all()
+
+
+@pytest.mark.parametrize("k", [1, 2, 3, 5, 15, 17, 34])
+@pytest.mark.parametrize("la,lb", [(0, 0), (1, 0), (0, 1), (1, 1), (2, 0), (1, 2)])
+@pytest.mark.parametrize("m,n,shift", [(1, 1, 0), (67, 130, 1), (129, 63, 3), (66, 65, 2)])
+def test_ragged_operands(oracle_lib, m, n, k, la, lb, shift):
+    """Rows that are no whole 16-byte parts, at every offset from them, along k (0), along m or n (1) and
+    with no unit stride (2): elements past a row's end, which hold NaN here, are not read into it."""
+    from densecore_amd import _native
+    print(f"[case] bmm ragged {m}x{n}x{k} A {la} B {lb} shift {shift}", flush=True)
+    rng = np.random.default_rng(m + n + k + shift)
+    batch = 3
+    a, b = rng.standard_normal((batch, m, k), dtype=np.float32), rng.standard_normal((batch, k, n), dtype=np.float32)
+
+    def operand(x, along):  # x is (batch, rows, k)
+        if along == 1:
+            x = x.transpose(0, 2, 1)
+        step = 2 if along == 2 else 1
+        pad = torch.full((batch, x.shape[1], shift + step * x.shape[2] + 5), float("nan"), device=DEV)
+        view = pad[:, :, shift:shift + step * x.shape[2]:step]
+        view.copy_(torch.from_numpy(np.ascontiguousarray(x)))
+        return view.transpose(1, 2) if along == 1 else view
+
+    got = _native._bmm(operand(a, la), operand(b.transpose(0, 2, 1), lb).transpose(1, 2)).cpu().numpy()
+    assert_f32(got, oracle_lib.bmm(a, b, b_k_contiguous=lb != 1), f"bmm {m}x{n}x{k}")
