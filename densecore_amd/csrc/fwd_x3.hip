@@ -533,12 +533,21 @@ hipError_t launch_rows(const FwdArgs &a, dim3 grid, bool split, hipStream_t st) 
                    : launch(fwd_x3_kernel<D, CAUSAL, MASK, false, false>, grid, block, st, a);
 }
 
+// How a grid of few query tiles splits the keys.  Pieces of 4 tiles of 32 keys, as for the float32
+// MFMA's tiles (of 64 keys up to head dim 32), are short ones here: on one MI355X, pieces of 4 -> one per
+// CU where that is estimated faster, B7 H2 L253 S1260 E32 22.8 -> 19.5 us (float32 MFMA 22.7), B8 H4 L128
+// S4096 E32 42.1 -> 33.7 (36.6), E64 42.7 -> 37.2, B1 H1 L128 S16384 E32 79.9 -> 46.8 (55.3), E64 80.2 ->
+// 49.5, E96 127 -> 82, causal B1 H16 L1000 E64 33.0 -> 30.1; one per CU wherever it fits, causal B1 H4 L4096
+// E32 62 -> 78.  Up to head dim 32, 256 keys are not worth a second launch (B1 H1 L864 S172 16.3 -> 13.8).
 template <int D>
 FwdSplitPlan plan(const AttnShape &s) {
+    if (D == 32 && s.S <= 256) return FwdSplitPlan{};
     const int64_t blocks = (int64_t)(s.L + kX3M - 1) / kX3M * s.B * s.H;
     const int64_t slots = split_slots(reinterpret_cast<const void *>(&fwd_x3_kernel<D, true, kNoMask, true, true>),
                                       kX3Threads, blocks);
-    return plan_split(s, kX3M, kX3BN, slots);
+    // Microseconds per tile in a workgroup with a CU to itself: L128 S16384 whole, 620 us at E32, 658 at
+    // E64, 1213 at E96.
+    return plan_split(s, kX3M, kX3BN, slots, D <= 64 ? 1.2f : 2.4f);
 }
 
 template <int D>
